@@ -26,6 +26,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "boys.hpp"
 #include "types.hpp"
 
@@ -50,9 +52,19 @@ __device__ __forceinline__ double wave_sum(double v) {
 // formed in FP64 and rounded once, and the integrals are widened to FP64
 // before digestion, whose sums and atomics stay in FP64.
 struct TileInfo {
-  PairRec bp, kp;
+  PairRec bp, kp;  // in kModeJK of kp only A, AB, fa, fb
   int bidx, kidx;
   bool active;
+};
+
+// What a tile is read from, as the kernel's restrict-qualified arguments
+// (nothing the kernel stores aliases them): wave-uniform records -- the tile,
+// the bra pair, the ket bucket's counts -- then come through the scalar unit
+// and are not read again after an atomic.
+struct TileSrc {
+  const PairRec* pairs;
+  const Tile* tiles;
+  KetPlanes ket;  // kModeJK
 };
 
 // The primitive-pair records a kernel of arithmetic type R reads: FP64
@@ -72,6 +84,24 @@ __device__ __forceinline__ const typename PrimOf<R>::T* prims_of(const PrimRec* 
   else return p32;
 }
 
+// One ket primitive pair of the lane, FP64 or FP32, from the planes (KP) or
+// from the records.
+template <typename R, bool KP>
+__device__ __forceinline__ typename PrimOf<R>::T load_ket_prim(
+    const KetPlanes& k, const typename PrimOf<R>::T* __restrict__ prim, int row, int lane_off) {
+  if constexpr (!KP) {
+    return prim[row + lane_off];
+  } else if constexpr (sizeof(R) == 8) {
+    const double2 a = (k.prim + row)[lane_off], b = (k.prim + k.nprims + row)[lane_off],
+                  c = (k.prim + 2 * static_cast<size_t>(k.nprims) + row)[lane_off];
+    return PrimRec{a.x, b.x, b.y, c.x, a.y, c.y};
+  } else {
+    const float4 a = (k.prim4 + row)[lane_off];
+    const float2 b = (k.prim2 + row)[lane_off];
+    return PrimRecF{a.x, a.y, a.z, a.w, b.x, b.y};
+  }
+}
+
 // Primitive loops: the ket primitive (per-lane, vector loads; with PF fetched
 // one iteration ahead) is the outer loop, the bra primitive the inner one, so
 // each ket record is read once per quartet.  The bra pair is wave-uniform, so
@@ -80,10 +110,11 @@ __device__ __forceinline__ const typename PrimOf<R>::T* prims_of(const PrimRec* 
 // what lets the compiler prove the loads unclobbered by the kernel's atomics
 // and issue them as scalar loads).  Records hold P - A relative to their pair's first centre; per lane
 // Q - A = (Q - C) - (A - C) once per ket primitive, then P - Q = (P - A) - (Q - A)
-// per primitive quartet.  `boys_tab` is the Boys grid in LDS.
+// per primitive quartet.  `boys_tab` is the Boys grid in LDS.  In kModeJK
+// ti.bp and ti.bidx are the caller's.
 template <int LA, int LB, int LC, int LD, int MODE, int BM, typename R, bool PF = true,
           int UNR = 1, bool BF = false>
-__device__ __forceinline__ void eri_compute(const EriArgs& a, const Tile t, const int lane,
+__device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, const int lane,
                                             TileInfo& ti,
                                             double (&out)[EriClass<LA, LB, LC, LD>::NOUT],
                                             const R* __restrict__ boys_tab,
@@ -91,12 +122,33 @@ __device__ __forceinline__ void eri_compute(const EriArgs& a, const Tile t, cons
   using C = EriClass<LA, LB, LC, LD>;
   using P = typename PrimOf<R>::T;
   constexpr int L = C::L;
+  constexpr bool KP = MODE == kModeJK;
   static_assert(BM == kBoysExact || sizeof(R) == 8, "compat Boys is FP64 only");
   ti.active = lane < t.count;
-  ti.kidx = t.ket0 + (ti.active ? lane : 0);
-  ti.bidx = (MODE == kModeDiag) ? ti.kidx : t.bra;
-  ti.bp = a.pairs[ti.bidx];
-  ti.kp = a.pairs[ti.kidx];
+  const int lane_off = ti.active ? lane : 0;  // an idle lane repeats the first
+  ti.kidx = t.ket0 + lane_off;
+  if constexpr (!KP) {
+    ti.bidx = (MODE == kModeDiag) ? ti.kidx : t.bra;
+    ti.bp = src.pairs[ti.bidx];
+    ti.kp = src.pairs[ti.kidx];
+  } else {
+    const KetPlanes& k = src.ket;
+    const double2 g0 = (k.geo + t.ket0)[lane_off], g1 = (k.geo + k.npairs + t.ket0)[lane_off];
+    const int2 f = (k.fn + t.ket0)[lane_off];
+    ti.kp.A[0] = g0.x;
+    ti.kp.A[1] = g0.y;
+    ti.kp.A[2] = g1.x;
+    ti.kp.fa = f.x;
+    ti.kp.fb = f.y;
+    if constexpr (LD > 0) {  // the HRR's C - D
+      const double2 g2 = (k.geo + 2 * static_cast<size_t>(k.npairs) + t.ket0)[lane_off];
+      ti.kp.AB[0] = g1.y;
+      ti.kp.AB[1] = g2.x;
+      ti.kp.AB[2] = g2.y;
+    } else {
+      ti.kp.AB[0] = ti.kp.AB[1] = ti.kp.AB[2] = 0.0;
+    }
+  }
   const PairRec& bp = ti.bp;
   const PairRec& kp = ti.kp;
 
@@ -107,7 +159,6 @@ __device__ __forceinline__ void eri_compute(const EriArgs& a, const Tile t, cons
   const R* __restrict__ table = boys_tab;
   // A - C in FP64, rounded once
   const R ACx = R(bp.A[0] - kp.A[0]), ACy = R(bp.A[1] - kp.A[1]), ACz = R(bp.A[2] - kp.A[2]);
-  const P* __restrict__ kprim = prim + kp.p0;
   // the bra pair's records: wave-uniform (said so, so that the address and the
   // trip count live in scalar registers), except in the diagonal mode
   const int bp0 = MODE == kModeDiag ? bp.p0 : __builtin_amdgcn_readfirstlane(bp.p0);
@@ -116,14 +167,27 @@ __device__ __forceinline__ void eri_compute(const EriArgs& a, const Tile t, cons
   const P* __restrict__ bprim = prim + bp0;
   // the ket pairs of a tile share their bucket, hence its primitive-pair count
   // and record stride: the ket loop is uniform too
-  const int knp = MODE == kModeDiag ? kp.np : __builtin_amdgcn_readfirstlane(kp.np);
-  const int kps = MODE == kModeDiag ? kp.ps : __builtin_amdgcn_readfirstlane(kp.ps);
-  P nxt = kprim[0];
+  // (in kModeJK and its lanes' first primitive records are consecutive too: the
+  // row of ket0 in a scalar register, the lane's place in it as an offset)
+  int knp, kps, row, row_off;
+  if constexpr (KP) {
+    const PairRec& k0 = src.pairs[t.ket0];
+    knp = k0.np;
+    kps = k0.ps;
+    row = k0.p0;
+    row_off = lane_off;
+  } else {
+    knp = MODE == kModeDiag ? kp.np : __builtin_amdgcn_readfirstlane(kp.np);
+    kps = MODE == kModeDiag ? kp.ps : __builtin_amdgcn_readfirstlane(kp.ps);
+    row = 0;
+    row_off = kp.p0;
+  }
+  P nxt = load_ket_prim<R, KP>(src.ket, prim, row, row_off);
   for (int j = 0; j < knp; ++j) {
     // with PF the next record is in flight during this iteration's work;
     // without, the load is issued here and other waves cover its latency
-    const P pk = PF ? nxt : kprim[j * kps];
-    if (PF && j + 1 < knp) nxt = kprim[(j + 1) * kps];
+    const P pk = PF ? nxt : load_ket_prim<R, KP>(src.ket, prim, row + j * kps, row_off);
+    if (PF && j + 1 < knp) nxt = load_ket_prim<R, KP>(src.ket, prim, row + (j + 1) * kps, row_off);
     const R zk = R(pk.zeta), kk = R(pk.kab), oo2e = R(pk.oo2z);
     const R QCx = R(pk.pax), QCy = R(pk.pay), QCz = R(pk.paz);
     const R QAx = QCx - ACx, QAy = QCy - ACy, QAz = QCz - ACz;
@@ -196,7 +260,9 @@ __device__ __forceinline__ const R* boys_src(const EriArgs& a) {
 // exponent field (integer operations in place of selects between doubles);
 // an inactive lane gets +0.
 __device__ __forceinline__ double symmetry_weight(const TileInfo& ti) {
-  const int e = (ti.bp.flags & 1) + (ti.kp.flags & 1) + (ti.bidx != ti.kidx ? 1 : 0);
+  // the shells of a pair differ if and only if their first functions do
+  const int e = (ti.bp.fa != ti.bp.fb ? 1 : 0) + (ti.kp.fa != ti.kp.fb ? 1 : 0) +
+                (ti.bidx != ti.kidx ? 1 : 0);
   const int hi = ti.active ? (1023 - 3 + e) << 20 : 0;
   return __hiloint2double(hi, 0);
 }
@@ -216,28 +282,53 @@ __device__ __forceinline__ double* at_off(double* base, unsigned boff) {
 //         K_bc += s (ab|cd) D_ad,  K_bd += s (ab|cd) D_ac.
 // add(row_is_b, row_component, column_function, value) receives each sum.
 // The bra functions fa, fb are wave-uniform: the density rows they index are
-// uniform bases, the ket columns fc, fd 32-bit byte offsets.
+// uniform bases, the ket columns fc, fd 32-bit byte offsets.  drows, if set:
+// those NA + NB rows in LDS (row r at drows + r * kw, column kc0 first): a
+// gather of 64 columns there meets a few bank conflicts, where in memory it
+// takes one L1 access for nearly every cache line of the row.
 template <int NA, int NB, int NC, int ND, typename Add>
 __device__ __forceinline__ void exchange_blocks(const double* __restrict__ D, int n, int fa,
                                                 int fb, int fc, int fd, const double* out,
-                                                double s, Add add) {
+                                                double s, Add add,
+                                                const double* drows = nullptr, int kw = 0,
+                                                int kc0 = 0) {
   double dbd[NB * ND], dbc[NB * NC], dad[NA * ND], dac[NA * NC];
-  const unsigned oc = static_cast<unsigned>(fc) * 8u, od = static_cast<unsigned>(fd) * 8u;
+  if (drows) {
+    const int oc = fc - kc0, od = fd - kc0;
 #pragma unroll
-  for (int ib = 0; ib < NB; ++ib) {
-    const double* __restrict__ row = D + static_cast<size_t>(fb + ib) * n;
+    for (int ib = 0; ib < NB; ++ib) {
+      const double* row = drows + (NA + ib) * kw;
 #pragma unroll
-    for (int id = 0; id < ND; ++id) dbd[ib * ND + id] = ld_off(row, od + 8u * id);
+      for (int id = 0; id < ND; ++id) dbd[ib * ND + id] = row[od + id];
 #pragma unroll
-    for (int ic = 0; ic < NC; ++ic) dbc[ib * NC + ic] = ld_off(row, oc + 8u * ic);
-  }
+      for (int ic = 0; ic < NC; ++ic) dbc[ib * NC + ic] = row[oc + ic];
+    }
 #pragma unroll
-  for (int ia = 0; ia < NA; ++ia) {
-    const double* __restrict__ row = D + static_cast<size_t>(fa + ia) * n;
+    for (int ia = 0; ia < NA; ++ia) {
+      const double* row = drows + ia * kw;
 #pragma unroll
-    for (int id = 0; id < ND; ++id) dad[ia * ND + id] = ld_off(row, od + 8u * id);
+      for (int id = 0; id < ND; ++id) dad[ia * ND + id] = row[od + id];
 #pragma unroll
-    for (int ic = 0; ic < NC; ++ic) dac[ia * NC + ic] = ld_off(row, oc + 8u * ic);
+      for (int ic = 0; ic < NC; ++ic) dac[ia * NC + ic] = row[oc + ic];
+    }
+  } else {
+    const unsigned oc = static_cast<unsigned>(fc) * 8u, od = static_cast<unsigned>(fd) * 8u;
+#pragma unroll
+    for (int ib = 0; ib < NB; ++ib) {
+      const double* __restrict__ row = D + static_cast<size_t>(fb + ib) * n;
+#pragma unroll
+      for (int id = 0; id < ND; ++id) dbd[ib * ND + id] = ld_off(row, od + 8u * id);
+#pragma unroll
+      for (int ic = 0; ic < NC; ++ic) dbc[ib * NC + ic] = ld_off(row, oc + 8u * ic);
+    }
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia) {
+      const double* __restrict__ row = D + static_cast<size_t>(fa + ia) * n;
+#pragma unroll
+      for (int id = 0; id < ND; ++id) dad[ia * ND + id] = ld_off(row, od + 8u * id);
+#pragma unroll
+      for (int ic = 0; ic < NC; ++ic) dac[ia * NC + ic] = ld_off(row, oc + 8u * ic);
+    }
   }
 #pragma unroll
   for (int ia = 0; ia < NA; ++ia)
@@ -329,15 +420,19 @@ __device__ __forceinline__ void coulomb_sums(const double* __restrict__ D, int n
 
 // Tile-granular kernel body: diagonal, tensor, and JK with global atomics.
 template <int LA, int LB, int LC, int LD, int MODE, int BM, typename R>
-__device__ __forceinline__ void eri_tile(const EriArgs& a, const Tile t, const int lane,
-                                         const R* __restrict__ boys_tab,
+__device__ __forceinline__ void eri_tile(const EriArgs& a, const TileSrc& src, const Tile t,
+                                         const int lane, const R* __restrict__ boys_tab,
                                          const typename PrimOf<R>::T* __restrict__ prim,
                                          const double* __restrict__ D) {
   using C = EriClass<LA, LB, LC, LD>;
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   TileInfo ti;
   double out[C::NOUT];
-  eri_compute<LA, LB, LC, LD, MODE, BM, R>(a, t, lane, ti, out, boys_tab, prim);
+  if constexpr (MODE == kModeJK) {
+    ti.bidx = t.bra;
+    ti.bp = src.pairs[t.bra];
+  }
+  eri_compute<LA, LB, LC, LD, MODE, BM, R>(src, t, lane, ti, out, boys_tab, prim);
   const int fc = ti.kp.fa, fd = ti.kp.fb;
   // the bra's functions are wave-uniform except in the diagonal mode
   const int fa = MODE == kModeDiag ? ti.bp.fa : __builtin_amdgcn_readfirstlane(ti.bp.fa);
@@ -407,10 +502,19 @@ __device__ __forceinline__ void eri_tile(const EriArgs& a, const Tile t, const i
 }
 
 template <int LA, int LB, int LC, int LD, int MODE, int BM, typename R>
-__global__ __launch_bounds__(256) void eri_kernel(const EriArgs a,
-                                                  const PrimRec* __restrict__ prims,
-                                                  const PrimRecF* __restrict__ prims_f,
-                                                  const double* __restrict__ D) {
+__global__ __launch_bounds__(256) void eri_kernel(
+    const EriArgs a, const PrimRec* __restrict__ prims, const PrimRecF* __restrict__ prims_f,
+    const double* __restrict__ D, const PairRec* __restrict__ pairs,
+    const Tile* __restrict__ tiles, const double2* __restrict__ kgeo,
+    const int2* __restrict__ kfn, const double2* __restrict__ kprim,
+    const float4* __restrict__ kprim4, const float2* __restrict__ kprim2) {
+  // Other modes than kModeJK read their records through the argument struct:
+  // with the restrict-qualified arrays the compat kernels of (dp|ds) and
+  // (dd|ds), whose 512 registers spill, returned a few wrong integrals
+  // (deterministic, the same instruction stream otherwise correct: a compiler
+  // fault), and no caller of theirs is bound by these loads.
+  const TileSrc src{MODE == kModeJK ? pairs : a.pairs, MODE == kModeJK ? tiles : a.tiles,
+                    KetPlanes{kgeo, kfn, kprim, kprim4, kprim2, a.ket.npairs, a.ket.nprims}};
   const typename PrimOf<R>::T* __restrict__ prim = prims_of<R>(prims, prims_f);
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -425,52 +529,69 @@ __global__ __launch_bounds__(256) void eri_kernel(const EriArgs a,
     // leaves the loop once its next index passes the end
     const int begin = a.tile_range[0], end = a.tile_range[1];
     for (int t = begin + w; t < end; t += gridDim.x * 4)
-      eri_tile<LA, LB, LC, LD, MODE, BM, R>(a, a.tiles[t], lane, boys_tab, prim, D);
+      eri_tile<LA, LB, LC, LD, MODE, BM, R>(a, src, src.tiles[t], lane, boys_tab, prim, D);
   } else {
     if (w >= a.ntiles) return;  // uniform per wave
-    eri_tile<LA, LB, LC, LD, MODE, BM, R>(a, a.tiles[w], lane, boys_tab, prim, D);
+    eri_tile<LA, LB, LC, LD, MODE, BM, R>(a, src, src.tiles[w], lane, boys_tab, prim, D);
   }
 }
 
 // LDS digestion: a fixed grid of workgroups drains chunks [range[0], range[1]).
 // Dynamic LDS holds the bra's K rows: (NA + NB) x kw doubles, columns
-// [kc0, kc0 + kw) (all nbf columns for one molecule).  W waves per workgroup
-// share them; OCC > 0 bounds the registers so that OCC waves fit a SIMD; PF
-// selects the one-ahead ket fetch, UNR the bra primitive pairs per inner
-// iteration, BF the branch-free Boys function (kLdsVariants lists the shapes).
+// [kc0, kc0 + kw) (all nbf columns for one molecule), and with d_rows the same
+// rows of the density after them.  W waves per workgroup share them; OCC > 0
+// bounds the registers so that OCC waves fit a SIMD; PF selects the one-ahead
+// ket fetch, UNR the bra primitive pairs per inner iteration, BF the
+// branch-free Boys function (kLdsVariants lists the shapes).
 template <int LA, int LB, int LC, int LD, int BM, typename R, int W, int OCC, bool PF,
           int UNR, bool BF>
 __global__ __launch_bounds__(64 * W, OCC > 0 ? OCC : 1) void eri_jk_lds_kernel(
-    const EriArgs a, const PrimRec* __restrict__ prims, const PrimRecF* __restrict__ prims_f,
-    const double* __restrict__ D, const double* __restrict__ Dp) {
+    const EriArgs a, int d_rows, const PrimRec* __restrict__ prims,
+    const PrimRecF* __restrict__ prims_f, const double* __restrict__ D,
+    const double* __restrict__ Dp, const PairRec* __restrict__ pairs,
+    const Tile* __restrict__ tiles, const Chunk* __restrict__ chunks,
+    const double2* __restrict__ kgeo, const int2* __restrict__ kfn,
+    const double2* __restrict__ kprim, const float4* __restrict__ kprim4,
+    const float2* __restrict__ kprim2) {
   const typename PrimOf<R>::T* __restrict__ prim = prims_of<R>(prims, prims_f);
+  const TileSrc src{pairs, tiles, KetPlanes{kgeo, kfn, kprim, kprim4, kprim2, a.ket.npairs,
+                                            a.ket.nprims}};
   using C = EriClass<LA, LB, LC, LD>;
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   extern __shared__ double krows[];
   __shared__ R boys_tab[boys_stage_size(C::L)];
   stage_boys<C::L>(boys_tab, boys_src<R>(a));
-  const size_t n = static_cast<size_t>(a.nbf);
   const int ni = a.nbf;
   const int kw = a.kw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int nrow = (NA + NB) * kw;
+  double* drows = d_rows ? krows + nrow : nullptr;
   const int begin = a.chunk_range[0], end = a.chunk_range[1];
   for (int ch = begin + blockIdx.x; ch < end; ch += gridDim.x) {  // block-uniform
-    const Chunk c = a.chunks[ch];
+    const Chunk c = chunks[ch];
     const int kc0 = a.pair_kc0 ? a.pair_kc0[c.bra] : 0;
-    for (int k = threadIdx.x; k < nrow; k += blockDim.x) krows[k] = 0.0;
+    TileInfo ti;
+    ti.bidx = c.bra;
+    ti.bp = pairs[c.bra];
+    const int fa = ti.bp.fa, fb = ti.bp.fb;
+#pragma unroll
+    for (int r = 0; r < NA + NB; ++r) {
+      const double* __restrict__ drow =
+          D + static_cast<size_t>(r < NA ? fa + r : fb + (r - NA)) * ni + kc0;
+      for (int k = threadIdx.x; k < kw; k += 64 * W) {
+        krows[r * kw + k] = 0.0;
+        if (drows) drows[r * kw + k] = drow[k];
+      }
+    }
     __syncthreads();
     double jab_acc[NA * NB];
 #pragma unroll
     for (int k = 0; k < NA * NB; ++k) jab_acc[k] = 0.0;
     for (int t = c.tb + wave; t < c.te; t += W) {  // wave-uniform
-      TileInfo ti;
       double out[C::NOUT];
-      eri_compute<LA, LB, LC, LD, kModeJK, BM, R, PF, UNR, BF>(a, a.tiles[t], lane, ti, out,
+      eri_compute<LA, LB, LC, LD, kModeJK, BM, R, PF, UNR, BF>(src, tiles[t], lane, ti, out,
                                                                boys_tab, prim);
-      const int fa = __builtin_amdgcn_readfirstlane(ti.bp.fa);
-      const int fb = __builtin_amdgcn_readfirstlane(ti.bp.fb);
       const int fc = ti.kp.fa, fd = ti.kp.fb;
       const double s = symmetry_weight(ti);
       double jab[NA * NB], jcd[NC * ND];
@@ -490,7 +611,8 @@ __global__ __launch_bounds__(64 * W, OCC > 0 ? OCC : 1) void eri_jk_lds_kernel(
                                         [&](bool rb, int comp, int col, double v) {
                                           atomicAdd(&krows[(rb ? NA + comp : comp) * kw + col - kc0],
                                                     v);
-                                        });
+                                        },
+                                        drows, kw, kc0);
       }
     }
     // bra Coulomb block: wave sums, one atomic per component per wave
@@ -502,13 +624,12 @@ __global__ __launch_bounds__(64 * W, OCC > 0 ? OCC : 1) void eri_jk_lds_kernel(
     }
     __syncthreads();
     // flush the K rows of a and b, contiguous along each row
-    const PairRec bp = a.pairs[c.bra];
-    for (int k = threadIdx.x; k < nrow; k += blockDim.x) {
-      const double v = krows[k];
-      if (v != 0.0) {
-        const int r = k / kw, col = kc0 + (k - r * kw);
-        const int row = r < NA ? bp.fa + r : bp.fb + (r - NA);
-        unsafeAtomicAdd(&a.K[row * n + col], v);
+#pragma unroll
+    for (int r = 0; r < NA + NB; ++r) {
+      double* krow = a.K + static_cast<size_t>(r < NA ? fa + r : fb + (r - NA)) * ni + kc0;
+      for (int k = threadIdx.x; k < kw; k += 64 * W) {
+        const double v = krows[r * kw + k];
+        if (v != 0.0) unsafeAtomicAdd(&krow[k], v);
       }
     }
     __syncthreads();
@@ -528,7 +649,8 @@ hipError_t eri_launch(const EriArgs& a, int blocks, hipStream_t s) {
     grid = static_cast<unsigned>((a.ntiles + 3) / 4);
   }
   hipLaunchKernelGGL((eri_kernel<LA, LB, LC, LD, MODE, BM, R>), dim3(grid), dim3(256), 0, s, a,
-                     a.prims, a.prims_f, a.D);
+                     a.prims, a.prims_f, a.D, a.pairs, a.tiles, a.ket.geo, a.ket.fn, a.ket.prim,
+                     a.ket.prim4, a.ket.prim2);
   return hipGetLastError();
 }
 
@@ -536,9 +658,25 @@ template <int LA, int LB, int LC, int LD, int BM, typename R, int W = 4, int OCC
           bool PF = true, int UNR = 1, bool BF = false>
 hipError_t eri_jk_lds_launch(const EriArgs& a, int blocks, hipStream_t s) {
   if (blocks <= 0) return hipSuccess;
-  const size_t lds = sizeof(double) * (ncart(LA) + ncart(LB)) * static_cast<size_t>(a.kw);
-  hipLaunchKernelGGL((eri_jk_lds_kernel<LA, LB, LC, LD, BM, R, W, OCC, PF, UNR, BF>), dim3(blocks),
-                     dim3(64 * W), lds, s, a, a.prims, a.prims_f, a.D, a.Dp);
+  const auto kernel = eri_jk_lds_kernel<LA, LB, LC, LD, BM, R, W, OCC, PF, UNR, BF>;
+  const size_t rows = sizeof(double) * (ncart(LA) + ncart(LB)) * static_cast<size_t>(a.kw);
+  // The density rows go to LDS beside the K rows unless that costs a third of
+  // the workgroups a CU would hold (by registers and LDS).  (H2O)_64 6-31G
+  // builds, FP64 / mixed: rows never in LDS 20.8 / 17.9 ms, always 20.0 / 17.8
+  // (the (11|10) kernels lose half their waves: 1.58 -> 2.17 ms), by this rule
+  // 19.4 / 16.9 ((10|00) 7.14 -> 6.25 ms FP64, 3.62 -> 3.09 FP32).
+  static const int reg_groups = [&] {
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 64 * W, 0) == hipSuccess ? n
+                                                                                             : 1;
+  }();
+  const size_t fixed = sizeof(R) * boys_stage_size(EriClass<LA, LB, LC, LD>::L);
+  const int with = std::min<int>(reg_groups, static_cast<int>(kLdsPerCu / (fixed + 2 * rows)));
+  const int without = std::min<int>(reg_groups, static_cast<int>(kLdsPerCu / (fixed + rows)));
+  const int d_rows = with > 0 && 3 * with >= 2 * without;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * W), d_rows ? 2 * rows : rows, s, a, d_rows,
+                     a.prims, a.prims_f, a.D, a.Dp, a.pairs, a.tiles, a.chunks, a.ket.geo,
+                     a.ket.fn, a.ket.prim, a.ket.prim4, a.ket.prim2);
   return hipGetLastError();
 }
 

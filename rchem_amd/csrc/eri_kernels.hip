@@ -14,6 +14,47 @@ using EriLaunchFn = hipError_t (*)(const EriArgs&, int, hipStream_t);
 
 #include "generated/eri_dispatch.inc"
 
+// The ket planes (types.hpp) of npairs pair records and nprims primitive
+// records, and the FP32 primitive records: one thread per record of either
+// kind.
+__global__ __launch_bounds__(256) void ket_planes_kernel(
+    const PairRec* __restrict__ pairs, int npairs, const PrimRec* __restrict__ prims, int nprims,
+    double2* __restrict__ geo, int2* __restrict__ fn, double2* __restrict__ prim,
+    float4* __restrict__ prim4, float2* __restrict__ prim2, PrimRecF* __restrict__ prims_f) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < npairs) {
+    const PairRec r = pairs[i];
+    const size_t n = static_cast<size_t>(npairs);
+    geo[i] = make_double2(r.A[0], r.A[1]);
+    geo[n + i] = make_double2(r.A[2], r.AB[0]);
+    geo[2 * n + i] = make_double2(r.AB[1], r.AB[2]);
+    fn[i] = make_int2(r.fa, r.fb);
+  }
+  if (i < nprims) {
+    const PrimRec r = prims[i];
+    const size_t n = static_cast<size_t>(nprims);
+    prim[i] = make_double2(r.zeta, r.kab);
+    prim[n + i] = make_double2(r.pax, r.pay);
+    prim[2 * n + i] = make_double2(r.paz, r.oo2z);
+    const PrimRecF f{static_cast<float>(r.zeta), static_cast<float>(r.pax),
+                     static_cast<float>(r.pay),  static_cast<float>(r.paz),
+                     static_cast<float>(r.kab),  static_cast<float>(r.oo2z)};
+    prims_f[i] = f;
+    prim4[i] = make_float4(f.zeta, f.pax, f.pay, f.paz);
+    prim2[i] = make_float2(f.kab, f.oo2z);
+  }
+}
+
+hipError_t ket_planes_launch(const PairRec* pairs, int npairs, const PrimRec* prims, int nprims,
+                             double2* geo, int2* fn, double2* prim, float4* prim4, float2* prim2,
+                             PrimRecF* prims_f, hipStream_t s) {
+  const int n = std::max(npairs, nprims);
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(ket_planes_kernel, dim3((n + 255) / 256), dim3(256), 0, s, pairs, npairs,
+                     prims, nprims, geo, fn, prim, prim4, prim2, prims_f);
+  return hipGetLastError();
+}
+
 // Jh[fa + ia, fb + ib] = Jp of pair p (each shell pair appears once, so the
 // writes do not collide); one thread per (pair, component).
 __global__ void jp_scatter_kernel(const PairRec* __restrict__ pairs, const double* __restrict__ Jp,

@@ -61,6 +61,9 @@ struct HostProgram {
 };
 #include "generated/eri_programs.inc"
 constexpr int kNumHostPrograms = sizeof(kHostPrograms) / sizeof(kHostPrograms[0]);
+hipError_t ket_planes_launch(const PairRec* pairs, int npairs, const PrimRec* prims, int nprims,
+                             double2* geo, int2* fn, double2* prim, float4* prim4, float2* prim2,
+                             PrimRecF* prims_f, hipStream_t s);
 hipError_t dpair_gather_launch(const PairRec* pairs, const double* D, const JpClass* cls,
                                const int* ncomp, int ncls, int npairs, double* Dp, int nbf,
                                hipStream_t s);
@@ -310,6 +313,7 @@ struct rchem_ctx {
   std::vector<Bucket> buckets[kNumPairClasses];
   int class_begin[kNumPairClasses + 1] = {0};
   DevBuf pairs_d, prims_d, prims_f_d;
+  DevBuf ket_geo_d, ket_fn_d, ket_prim_d, ket_prim4_d, ket_prim2_d;  // KetPlanes of the pair list
   DevBuf alpha_d;  // exponent of the first shell of every primitive pair (prims layout)
 
   // tiles for a threshold
@@ -733,18 +737,21 @@ int layout_pairs(rchem_ctx* ctx, const std::vector<PairHost>& sel, double prim_e
   if (!prims.empty())
     HIPC(hipMemcpyAsync(ctx->prims_d.p, prims.data(), sizeof(PrimRec) * prims.size(),
                         hipMemcpyHostToDevice, ctx->stream));
-  std::vector<PrimRecF> primsf(prims.size());
-  for (size_t k = 0; k < prims.size(); ++k) {
-    const PrimRec& r = prims[k];
-    primsf[k] = PrimRecF{static_cast<float>(r.zeta), static_cast<float>(r.pax),
-                         static_cast<float>(r.pay), static_cast<float>(r.paz),
-                         static_cast<float>(r.kab), static_cast<float>(r.oo2z)};
-  }
-  HIPC(ctx->prims_f_d.ensure(sizeof(PrimRecF) * std::max<size_t>(primsf.size(), 1)));
-  if (!primsf.empty())
-    HIPC(hipMemcpyAsync(ctx->prims_f_d.p, primsf.data(), sizeof(PrimRecF) * primsf.size(),
-                        hipMemcpyHostToDevice, ctx->stream));
-  HIPC(hipStreamSynchronize(ctx->stream));  // primsf is a local
+  // the ket planes and the FP32 records are formed on the device
+  const size_t npr = std::max<size_t>(ctx->pairs.size(), 1), npp = std::max<size_t>(prims.size(), 1);
+  HIPC(ctx->prims_f_d.ensure(sizeof(PrimRecF) * npp));
+  HIPC(ctx->ket_geo_d.ensure(sizeof(double2) * 3 * npr));
+  HIPC(ctx->ket_fn_d.ensure(sizeof(int2) * npr));
+  HIPC(ctx->ket_prim_d.ensure(sizeof(double2) * 3 * npp));
+  HIPC(ctx->ket_prim4_d.ensure(sizeof(float4) * npp));
+  HIPC(ctx->ket_prim2_d.ensure(sizeof(float2) * npp));
+  HIPC(ket_planes_launch(ctx->pairs_d.as<PairRec>(), static_cast<int>(ctx->pairs.size()),
+                         ctx->prims_d.as<PrimRec>(), static_cast<int>(prims.size()),
+                         ctx->ket_geo_d.as<double2>(), ctx->ket_fn_d.as<int2>(),
+                         ctx->ket_prim_d.as<double2>(), ctx->ket_prim4_d.as<float4>(),
+                         ctx->ket_prim2_d.as<float2>(), ctx->prims_f_d.as<PrimRecF>(),
+                         ctx->stream));
+  HIPC(hipStreamSynchronize(ctx->stream));  // prims is a local
   return RCHEM_OK;
 }
 
@@ -1375,6 +1382,13 @@ EriArgs base_args(const rchem_ctx* ctx) {
   a.nbf = ctx->nbf;
   a.boys_table = ctx->boys_d.as<double>();
   a.boys_table_f = ctx->boys_f_d.as<float>();
+  a.ket.geo = ctx->ket_geo_d.as<double2>();
+  a.ket.fn = ctx->ket_fn_d.as<int2>();
+  a.ket.prim = ctx->ket_prim_d.as<double2>();
+  a.ket.prim4 = ctx->ket_prim4_d.as<float4>();
+  a.ket.prim2 = ctx->ket_prim2_d.as<float2>();
+  a.ket.npairs = static_cast<int>(ctx->pairs.size());
+  a.ket.nprims = static_cast<int>(ctx->nprims);
   return a;
 }
 

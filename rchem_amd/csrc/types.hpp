@@ -45,6 +45,27 @@ struct PrimRecF {
   float zeta, pax, pay, paz, kab, oo2z;
 };
 
+// The ket side of a Fock build reads its pair and primitive records as planes:
+// 64 lanes hold 64 consecutive ket pairs, so a plane of 16-byte elements is
+// read as 1 KB of consecutive memory (8 cache lines), where the same fields
+// out of 72- and 48-byte records touch 36 and 24 lines for every 16 bytes a
+// lane takes.  Those line accesses kept the vector L1 of the s/p kernels busy
+// for all of their time on (H2O)_64 (texture-data unit 0.86-1.00, 0.7-1.35
+// cache accesses per cycle and CU, VALU 0.6).  Planes of n elements each, one
+// after the other (geo, prim) or one array each:
+//   geo:   (A_x, A_y), (A_z, AB_x), (AB_y, AB_z)   of pair p at p, n + p, 2n + p
+//   fn:    (fa, fb); the shells differ if and only if fa != fb
+//   prim:  (zeta, K_ab), (PA_x, PA_y), (PA_z, 1/2zeta)   of primitive pair r
+//   prim4, prim2: the FP32 record as (zeta, PA) and (K_ab, 1/2zeta)
+struct KetPlanes {
+  const double2* geo;
+  const int2* fn;
+  const double2* prim;
+  const float4* prim4;
+  const float2* prim2;
+  int npairs, nprims;
+};
+
 // A wavefront's work: one bra pair against up to 64 consecutive ket pairs of
 // one bucket (uniform primitive-pair count across the wave).
 struct Tile {
@@ -78,6 +99,7 @@ struct LdsVariant {
 constexpr LdsVariant kLdsVariants[] = {
     {4, 0, 1, 1, 0}, {4, 0, 0, 1, 0}, {8, 0, 1, 1, 0}, {8, 0, 0, 1, 0}, {8, 6, 0, 1, 0},
     {8, 8, 0, 1, 0}, {16, 0, 0, 1, 0}, {8, 0, 0, 2, 1}, {4, 0, 0, 2, 1}, {8, 0, 0, 1, 1}};
+constexpr size_t kLdsPerCu = 160 * 1024;
 constexpr int kNumLdsVariants = sizeof(kLdsVariants) / sizeof(kLdsVariants[0]);
 
 // Pair-indexed Coulomb accumulators: component k of pair p (pair class X) is
@@ -115,6 +137,7 @@ struct EriArgs {
   // and kw the largest molecule's function count
   int kw;
   const int* pair_kc0;
+  KetPlanes ket;     // kModeJK: the ket side's records
   // kModeGrad (wave-cooperative kernel): exponent of the first shell of each
   // primitive pair (same layout as prims), atoms of each pair's two shells,
   // and the 3 x natom gradient accumulated into
