@@ -170,12 +170,20 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
   // (in kModeJK and its lanes' first primitive records are consecutive too: the
   // row of ket0 in a scalar register, the lane's place in it as an offset)
   int knp, kps, row, row_off;
+  int i0 = 0, i1 = bnp;  // bra primitives
   if constexpr (KP) {
     const PairRec& k0 = src.pairs[t.ket0];
     knp = k0.np;
     kps = k0.ps;
     row = k0.p0;
     row_off = lane_off;
+    if (t.pad != 0) {  // a part of the quartets' primitives
+      i0 = t.pad & 255;
+      i1 = (t.pad >> 8) & 255;
+      const int j0 = (t.pad >> 16) & 255;
+      knp = ((t.pad >> 24) & 255) - j0;
+      row += j0 * kps;
+    }
   } else {
     knp = MODE == kModeDiag ? kp.np : __builtin_amdgcn_readfirstlane(kp.np);
     kps = MODE == kModeDiag ? kp.ps : __builtin_amdgcn_readfirstlane(kp.ps);
@@ -211,9 +219,9 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
                          roe * PQx, roe * PQy, roe * PQz, R(pb.oo2z), oo2e, R(0.5) * ooze, roz,
                          roe, PQx, PQy, PQz, acc);
     };
-    int i = 0;
+    int i = i0;
     if constexpr (UNR == 2) {
-      for (; i + 1 < bnp; i += 2) {
+      for (; i + 1 < i1; i += 2) {
         const P pb0 = bprim[i * bps];
         const P pb1 = bprim[(i + 1) * bps];
         prim_quartet(pb0);
@@ -226,9 +234,9 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
       // FP64 keeps the plain loop: there this form measured no faster, and
       // in the spilling L = 5, 6 per-lane kernels (quartet mode) it gave wrong
       // integrals, a cause not found; the FP32 kernels stop at L = 4.
-      if (bnp > 0) {
-        P cur = bprim[0];
-        for (; i + 1 < bnp; ++i) {
+      if (i < i1) {
+        P cur = bprim[i * bps];
+        for (; i + 1 < i1; ++i) {
           const P nxt_b = bprim[(i + 1) * bps];
           prim_quartet(cur);
           cur = nxt_b;
@@ -236,7 +244,7 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
         prim_quartet(cur);
       }
     } else {
-      for (; i < bnp; ++i) prim_quartet(bprim[i * bps]);
+      for (; i < i1; ++i) prim_quartet(bprim[i * bps]);
     }
   }
 

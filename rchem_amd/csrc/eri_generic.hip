@@ -286,6 +286,7 @@ __global__ __launch_bounds__(64 * W) void eri_generic_kernel(const EriArgs a,
   for (int ti = begin + static_cast<int>(blockIdx.x) * W + wave; ti < end;
        ti += static_cast<int>(gridDim.x) * W) {
     const Tile t = a.tiles[ti];
+    if (MODE == kModeJK && !first_part(t.pad)) continue;  // the first part does the whole quartet
     for (int i = 0; i < t.count; ++i) {
       const int kidx = t.ket0 + i;
       const int bidx = (MODE == kModeDiag) ? kidx : t.bra;

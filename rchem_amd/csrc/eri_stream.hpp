@@ -116,6 +116,7 @@ __global__ __launch_bounds__(64 * W, 1) void eri_stream_kernel(
   for (int ti = begin + static_cast<int>(blockIdx.x) * W + wave; ti < end;
        ti += static_cast<int>(gridDim.x) * W) {
     const Tile t = tiles[__builtin_amdgcn_readfirstlane(ti)];
+    if (MODE == kModeJK && !first_part(t.pad)) continue;  // the first part does the whole quartet
     for (int qi = 0; qi < t.count; ++qi) {
       const int kidx = __builtin_amdgcn_readfirstlane(t.ket0 + qi);
       const int bidx = __builtin_amdgcn_readfirstlane((MODE == kModeDiag) ? kidx : t.bra);

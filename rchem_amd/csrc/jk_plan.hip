@@ -129,9 +129,11 @@ __global__ void plan_kernel(const PlanArgs a) {
     a.lo[t] = lo;
     a.mid[t] = mid;
     a.hi[t] = hi;
-    a.cnt64[t] = (mid - lo + 63) >> 6;
-    a.cnt32[t] = (hi - mid + 63) >> 6;
-    const double npp = static_cast<double>(a.pairs[i].np) * bk.z;
+    const int np = a.pairs[i].np;
+    const int parts = PrimSplit(np, bk.z, pc.limit).parts();
+    a.cnt64[t] = ((mid - lo + 63) >> 6) * parts;
+    a.cnt32[t] = ((hi - mid + 63) >> 6) * parts;
+    const double npp = static_cast<double>(np) * bk.z;
     q64 = mid - lo;
     q32 = hi - mid;
     p64 = q64 * npp;
@@ -168,12 +170,19 @@ __global__ void expand_kernel(const PlanArgs a, const int* __restrict__ off64,
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= a.ntasks) return;
   const PlanClass pc = a.classes[class_of_task(a, t)];
-  const int i = pc.bra_begin + (t - pc.task_begin) / pc.nbk;
+  const int local = t - pc.task_begin;
+  const int i = pc.bra_begin + local / pc.nbk;
   const int lo = a.lo[t], mid = a.mid[t], hi = a.hi[t];
+  const PrimSplit sp(a.pairs[i].np, a.buckets[pc.bk_off + local % pc.nbk].z, pc.limit);
+  const int parts = sp.parts();
   int o = off64[t];
-  for (int k = lo; k < mid && o < cap; k += 64, ++o) tiles64[o] = Tile{i, k, min(64, mid - k), 0};
+  for (int k = lo; k < mid; k += 64)
+    for (int p = 0; p < parts && o < cap; ++p, ++o)
+      tiles64[o] = Tile{i, k, min(64, mid - k), sp.pad(p)};
   o = off32[t];
-  for (int k = mid; k < hi && o < cap; k += 64, ++o) tiles32[o] = Tile{i, k, min(64, hi - k), 0};
+  for (int k = mid; k < hi; k += 64)
+    for (int p = 0; p < parts && o < cap; ++p, ++o)
+      tiles32[o] = Tile{i, k, min(64, hi - k), sp.pad(p)};
 }
 
 __device__ __forceinline__ int class_of_unit(const PlanArgs& a, int u) {

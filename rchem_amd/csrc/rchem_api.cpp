@@ -1095,6 +1095,24 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
   return RCHEM_OK;
 }
 
+// Primitive quartets a tile of the class may take one after the other
+// (PrimSplit), `iters` its tiles' primitive quartets in all: half of what one of
+// the chip's 1024 SIMDs gets of the class, and not below what the digestion of
+// a part costs (16 primitive quartets for (ss|ss), less where a primitive
+// quartet is more work).  Build times in ms with tiles whole, and with the
+// share taken as iters / 512, 1024, 2048, 4096, 8192 ((ss|ss) floor 16 or 32):
+// (H2O)_8 6-31G through host buffers 1.37: 0.93, 0.79, 0.80, 0.84, 1.03;
+// (H2O)_12 gradient with its SCF 81.7: 77.6, 72.3, 72.6, -, -; 48 molecules'
+// SCF 108.1: 108.2, 108.0, 106.5, -, -; water STO-3G 0.38: 0.20, 0.20, 0.19,
+// 0.19, 0.19.  (H2O)_64: never below a tile's length, 19.5 either way.
+int split_limit(const QClass& qc, double iters) {
+  const int floor = 16 >> std::min(2, qc.la + qc.lb + qc.lc + qc.ld);
+  return std::max(floor, static_cast<int>(std::min(1e9, iters / 2048.0)));
+}
+// A workgroup takes a chunk's tiles in turn, so a class's chunks are at most its
+// tiles / 1024 (at least 8): (H2O)_8 1.06 -> 0.84 ms, water 0.26 -> 0.19.
+constexpr double kMinChunks = 1024.0;
+
 // Device-planner tables for threshold tau: classes, buckets, capacities and
 // the FP64 statistics (exact for all-FP64 builds).
 constexpr double kPassTiles = 67108864.0;  // 2^26 tiles (1 GiB per tile list) per pass
@@ -1133,6 +1151,8 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
     bra_cap[c].assign(ctx->class_begin[qc.X + 1] - ctx->class_begin[qc.X], 0.0);
   }
   for (auto& qc : ctx->qclasses) qc.quartets = qc.prim_quartets = qc.flops = 0.0;
+  std::vector<int> npmax(nq, 0);  // most primitive quartets to a quartet
+  std::vector<double> iters(nq, 0.0);  // primitive quartets of whole tiles (64 lanes)
   for_each_task(ctx, tau, [&](int X, int Y, int i, int b, int lo, int hi) {
     const int c = cls_index[X * kNumPairClasses + Y];
     if (c < 0) return;
@@ -1140,10 +1160,36 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
     bra_cap[c][i - ctx->class_begin[X]] += (cnt + 63) / 64 + 1;
     if (cnt <= 0) return;
     QClass& qc = ctx->qclasses[c];
-    const double pq = static_cast<double>(cnt) * ctx->pairs[i].np * ctx->buckets[Y][b].np;
+    const int npp = ctx->pairs[i].np * ctx->buckets[Y][b].np;
     qc.quartets += cnt;
-    qc.prim_quartets += pq;
+    qc.prim_quartets += static_cast<double>(cnt) * npp;
+    npmax[c] = std::max(npmax[c], npp);
+    iters[c] += static_cast<double>((cnt + 63) / 64) * npp;
   });
+  // Split tiles (PrimSplit) where a class's longest tile is longer than its
+  // waves' share of the class; the tiles reserved are then counted again.
+  std::vector<int> limit(nq, 0);
+  bool split = false;
+  for (size_t c = 0; c < nq; ++c) {
+    const QClass& qc = ctx->qclasses[c];
+    ClassKernel k;
+    if (qc.quartets > 0)
+      TRY(class_kernel(ctx, qc.la, qc.lb, qc.lc, qc.ld, kModeJK, kBoysExact, 0, &k));
+    if (!k.fn) continue;  // the other engines spread a quartet over a wave
+    limit[c] = split_limit(qc, iters[c]);
+    if (limit[c] >= npmax[c]) limit[c] = 0;
+    if (limit[c] > 0) {
+      split = true;
+      std::fill(bra_cap[c].begin(), bra_cap[c].end(), 0.0);
+    }
+  }
+  if (split)
+    for_each_task(ctx, tau, [&](int X, int Y, int i, int b, int lo, int hi) {
+      const int c = cls_index[X * kNumPairClasses + Y];
+      if (c < 0 || limit[c] == 0) return;
+      const int parts = PrimSplit(ctx->pairs[i].np, ctx->buckets[Y][b].np, limit[c]).parts();
+      bra_cap[c][i - ctx->class_begin[X]] += ((hi - lo + 63) / 64 + 1.0) * parts;
+    });
   for (size_t c = 0; c < nq; ++c) {
     QClass& qc = ctx->qclasses[c];
     int fh = 0;
@@ -1161,6 +1207,13 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
                                                     class_name(qc.la, qc.lb, qc.lc, qc.ld) +
                                                     " not served by this library");
     }
+  }
+  // chunks short enough that a class has some thousand of them
+  std::vector<int> chunk_most(nq);
+  for (size_t c = 0; c < nq; ++c) {
+    double tiles = 0.0;
+    for (const double x : bra_cap[c]) tiles += x;
+    chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(8.0, tiles / kMinChunks)));
   }
   // segments and passes
   rchem_ctx::Pass cur{0, 0, 0, 0, 0, 0, 0};
@@ -1186,8 +1239,9 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
     pc.unit_begin = cur.units;
     const ClassTune t64 = tune_for(ctx, qc.la, qc.lb, qc.lc, qc.ld, 0);
     const ClassTune t32 = tune_for(ctx, qc.la, qc.lb, qc.lc, qc.ld, 1);
-    pc.chunk64 = t64.chunk_tiles;
-    pc.chunk32 = t32.chunk_tiles;
+    pc.limit = limit[c];
+    pc.chunk64 = std::min(t64.chunk_tiles, chunk_most[c]);
+    pc.chunk32 = std::min(t32.chunk_tiles, chunk_most[c]);
     pc.order = (ket_order_of(ctx, t64) ? 1 : 0) | (ket_order_of(ctx, t32) ? 2 : 0);
     cur.order |= pc.order;
     ctx->pclasses.push_back(pc);

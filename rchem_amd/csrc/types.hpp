@@ -72,8 +72,42 @@ struct Tile {
   int bra;
   int ket0;
   int count;
+  // kModeJK: 0, or the primitive pairs this tile takes of its quartets, bra
+  // [i0, i1) and ket [j0, j1), as i0 | i1 << 8 | j0 << 16 | j1 << 24;
+  // kModeQuartet: where the quartet's block begins in the output
   int pad;
 };
+
+// A quartet's primitive loops are one lane's serial chain: 1296 primitive
+// quartets for two 6-31G oxygen cores, ~0.25 us each, and a small system's
+// build lasted as long as its longest tiles ((00|00) of (H2O)_8: 0.30 ms, of
+// which the work at full occupancy is 0.03).  Where a class has too little work
+// to hide that, its tiles are cut into parts of at most `limit` primitive
+// quartets (0: never), each digested on its own: J and K are sums over
+// primitives.  Bra primitives are cut first (the ket records are then read
+// once a part), ket primitives where one bra primitive still has too many.
+struct PrimSplit {
+  int nb, nk;        // primitive pairs of the bra and the ket
+  int bparts, kparts;
+  __host__ __device__ PrimSplit(int nb_, int nk_, int limit)
+      : nb(nb_), nk(nk_), bparts(1), kparts(1) {
+    if (limit <= 0 || nb * nk <= limit) return;
+    const int per = limit > nk ? limit / nk : 1;  // bra primitives to a part
+    bparts = (nb + per - 1) / per;
+    if (nk > limit) kparts = (nk + limit - 1) / limit;
+  }
+  __host__ __device__ int parts() const { return bparts * kparts; }
+  // Tile::pad of part p
+  __host__ __device__ int pad(int p) const {
+    if (bparts * kparts == 1) return 0;
+    const int b = p / kparts, k = p % kparts;
+    return (nb * b / bparts) | (nb * (b + 1) / bparts) << 8 | (nk * k / kparts) << 16 |
+           (nk * (k + 1) / kparts) << 24;
+  }
+};
+// A whole quartet, or the first part of a split one: what a kernel that cannot
+// take a part works on (it does the whole quartet then and skips the others).
+__host__ __device__ inline bool first_part(int pad) { return (pad & 0x00ff00ff) == 0; }
 
 // A block's work in LDS-digestion mode: tiles [tb, te) of one bra pair.
 struct Chunk {
@@ -196,6 +230,7 @@ struct PlanClass {
   int unit_begin;          // first bra unit; units = bra - bra_begin
   int chunk64, chunk32;    // tiles per LDS-digestion chunk, FP64 and FP32 lists
   int order;               // bit 0 / 1: FP64 / FP32 chunks ordered by first ket pair
+  int limit;               // PrimSplit's limit
 };
 
 struct PlanArgs {
