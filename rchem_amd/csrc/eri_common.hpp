@@ -526,7 +526,7 @@ __global__ __launch_bounds__(256) void eri_kernel(
   const typename PrimOf<R>::T* __restrict__ prim = prims_of<R>(prims, prims_f);
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  __shared__ R boys_tab[boys_stage_size(EriClass<LA, LB, LC, LD>::L)];
+  __shared__ __align__(16) R boys_tab[boys_stage_size(EriClass<LA, LB, LC, LD>::L, sizeof(R) == 8)];
   stage_boys<EriClass<LA, LB, LC, LD>::L>(boys_tab, boys_src<R>(a));
   __syncthreads();
   // the wave index is wave-uniform; saying so lets the tile, the bra pair and
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(64 * W, OCC > 0 ? OCC : 1) void eri_jk_lds_kernel(
   using C = EriClass<LA, LB, LC, LD>;
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
   extern __shared__ double krows[];
-  __shared__ R boys_tab[boys_stage_size(C::L)];
+  __shared__ __align__(16) R boys_tab[boys_stage_size(C::L, sizeof(R) == 8)];
   stage_boys<C::L>(boys_tab, boys_src<R>(a));
   const int ni = a.nbf;
   const int kw = a.kw;
@@ -678,7 +678,7 @@ hipError_t eri_jk_lds_launch(const EriArgs& a, int blocks, hipStream_t s) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 64 * W, 0) == hipSuccess ? n
                                                                                              : 1;
   }();
-  const size_t fixed = sizeof(R) * boys_stage_size(EriClass<LA, LB, LC, LD>::L);
+  const size_t fixed = sizeof(R) * boys_stage_size(EriClass<LA, LB, LC, LD>::L, sizeof(R) == 8);
   const int with = std::min<int>(reg_groups, static_cast<int>(kLdsPerCu / (fixed + 2 * rows)));
   const int without = std::min<int>(reg_groups, static_cast<int>(kLdsPerCu / (fixed + rows)));
   const int d_rows = with > 0 && 3 * with >= 2 * without;

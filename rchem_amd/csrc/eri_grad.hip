@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void eri_grad_kernel(const EriArgs a) {
   constexpr int NA = nc1(LA), NB = nc1(LB), NC = nc1(LC), ND = nc1(LD);
   constexpr int NQ = NA * NB * NC * ND;
   static_assert(G::NOUT == 9 * NQ, "gradient outputs: 3 centres x 3 axes x components");
-  __shared__ double boys_tab[kBoysStageSize];
+  __shared__ __align__(16) double boys_tab[boys_stage_size(L)];
   stage_boys<L>(boys_tab, a.boys_table);
   __syncthreads();
   const int lane = threadIdx.x & 63;

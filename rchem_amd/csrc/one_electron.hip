@@ -141,7 +141,7 @@ template <int LA, int LB>
 __global__ __launch_bounds__(128) void one_electron_kernel(const OneElArgs a) {
   constexpr int L = LA + LB;
   constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2;
-  __shared__ double boys_tab[kBoysStageSize];
+  __shared__ __align__(16) double boys_tab[boys_stage_size(L)];
   stage_boys<L>(boys_tab, a.boys_table);
   __syncthreads();
   const int c = 3 * LA + LB;
@@ -502,7 +502,7 @@ __device__ __forceinline__ double wave_sum_1(double v) {
 // atomic per component instead of 64 on the same few addresses).
 template <int LA, int LB>
 __global__ __launch_bounds__(128) void one_electron_grad_kernel(const OneElGradArgs a) {
-  __shared__ double boys_tab[kBoysStageSize];
+  __shared__ __align__(16) double boys_tab[boys_stage_size(LA + LB + 1)];
   stage_boys<LA + LB + 1>(boys_tab, a.boys_table);
   __syncthreads();
   const int c_cls = 3 * LA + LB;
