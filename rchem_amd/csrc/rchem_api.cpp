@@ -96,6 +96,9 @@ hipError_t diis_extrapolate_launch(const double* Fs, size_t n2, const ScfDevStat
 hipError_t scf_commit_launch(double* D, const double* Dn, size_t n2, ScfDevState* st,
                              const double* coef, int steps, double tol, double damping,
                              hipStream_t s);
+hipError_t density_small_launch(const double* F, const double* X, int ld, int nmax, const int* nb,
+                                int nocc1, const int* nocc, int count, double* D, double* flag,
+                                hipStream_t s);
 hipError_t batch_pack(const double* A, size_t n, const int* f0, const int* nb, int nmax, int nbatch,
                       double pad, double* out, hipStream_t s);
 hipError_t batch_unpack(const double* in, int nmax, const int* f0, const int* nb, int nbatch,
@@ -2653,6 +2656,14 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
   // kPurifyMax steps (no gap at the Fermi level), and the eigensolver takes over.
   constexpr int kPurifyMax = 200;
   constexpr double kPurifyTol = 1e-9;
+  // Up to kDensityMaxN functions the whole density, F' and projector included,
+  // is one launch (scf_density.hip); it reads as a purification of kSmallSteps
+  // steps that converged in the first or not at all.
+  const bool small = n <= kDensityMaxN;
+  constexpr int kSmallSteps = 3;
+  DevBuf dflag;
+  HIPC(dflag.ensure(sizeof(double) * 2 * kSmallSteps));
+  if (small) HIPC(fill_launch(dflag.as<double>(), 2 * kSmallSteps, 1.0, ctx->stream));
   DevBuf dP, dP2, dP3, dpl, dph, dpar;
   if (opts->purify) {
     for (DevBuf* b : {&dP, &dP2, &dP3}) HIPC(b->ensure(n2 * sizeof(double)));
@@ -2712,6 +2723,18 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
   // eigensolver formed it
   auto density = [&](const double* Fm, double* Dout, int* psteps) -> int {
     if (psteps) *psteps = 0;
+    if (small) {
+      HIPC(density_small_launch(Fm, dX.as<double>(), n, n, nullptr, opts->nocc, nullptr, 1, Dout,
+                                dflag.as<double>(), ctx->stream));
+      double f[2] = {0.0, 1.0};
+      HIPC(hipMemcpyAsync(f, dflag.p, sizeof(f), hipMemcpyDeviceToHost, ctx->stream));
+      HIPC(hipStreamSynchronize(ctx->stream));
+      if (f[1] == 0.0) {
+        if (psteps && opts->purify) *psteps = kSmallSteps;
+        return RCHEM_OK;
+      }
+      // no gap: the purification in memory (if asked for) and the eigensolver
+    }
     TRY(orthogonalise(Fm));
     if (opts->purify) {
       int steps = 0;
@@ -2816,6 +2839,13 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
     // the density of F_x by a fixed number of purification steps, committed
     // by the device if tr(P - P^2) was below kPurifyTol two steps before the end
     auto back_fixed = [&](int steps) -> int {
+      if (small) {
+        HIPC(density_small_launch(dFx.as<double>(), dX.as<double>(), n, n, nullptr, opts->nocc,
+                                  nullptr, 1, dDn.as<double>(), dflag.as<double>(), ctx->stream));
+        HIPC(scf_commit_launch(dD.as<double>(), dDn.as<double>(), n2, st, dflag.as<double>(),
+                               kSmallSteps, kPurifyTol, opts->damping, ctx->stream));
+        return RCHEM_OK;
+      }
       TRY(orthogonalise(dFx.as<double>()));
       HIPC(purify_start_launch(dFp.as<double>(), n, opts->nocc, dpl.as<double>(),
                                dph.as<double>(), dpar.as<double>(), dP.as<double>(), ctx->stream));
@@ -3214,7 +3244,25 @@ int batch_chunk(rchem_ctx* ctx, int m0, int m1, const int* natom, const int* Z,
   HIPC(hipStreamSynchronize(st));
   dS.release();  // its blocks live on in dSp
   // density from a padded Fock batch: F' = X^T F X, eigh, C = X C', D = C_occ C_occ^T
+  DevBuf dflag;
+  HIPC(dflag.ensure(sizeof(double) * 2 * B));
+  std::vector<double> flags(2 * static_cast<size_t>(B));
   auto density_b = [&](const double* Fb) -> int {
+    if (nm <= kDensityMaxN) {
+      // every molecule's in one launch, unless one of them has no gap
+      HIPC(density_small_launch(Fb, dX.as<double>(), nm, nm, dnb.as<int>(), 0, dnocc.as<int>(), Bs,
+                                dDb.as<double>(), dflag.as<double>(), st));
+      HIPC(hipMemcpyAsync(flags.data(), dflag.p, sizeof(double) * 2 * Bs, hipMemcpyDeviceToHost,
+                          st));
+      HIPC(hipStreamSynchronize(st));
+      bool good = true;
+      for (int s = 0; s < Bs; ++s) good = good && flags[2 * s + 1] == 0.0;
+      if (good) {
+        HIPC(batch_unpack(dDb.as<double>(), nm, df0.as<int>(), dnb.as<int>(), Bs, n,
+                          dD.as<double>(), st));
+        return RCHEM_OK;
+      }
+    }
     BLASC(gemm_b(rocblas_operation_none, rocblas_operation_none, Fb, dX.as<double>(), dT1.as<double>()));
     BLASC(gemm_b(rocblas_operation_transpose, rocblas_operation_none, dX.as<double>(),
                  dT1.as<double>(), dW.as<double>()));

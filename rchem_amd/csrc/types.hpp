@@ -323,6 +323,10 @@ struct ScfDevParams {
   int fp64;                    // the build being replayed is the all-FP64 one
   int pad;
 };
+// Functions up to which a density is formed by one workgroup (scf_density.hip):
+// the matrix in its LDS, 128 x 130 doubles.
+constexpr int kDensityMaxN = 128;
+
 constexpr int kDiisBlocks = 240;  // fixed grid of the dot-product pass: fixed summation order
 
 }  // namespace rchem
