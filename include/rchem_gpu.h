@@ -256,9 +256,9 @@ typedef struct rchem_scf_opts {
                           has no gap.  Single-molecule SCF and gradient (whose
                           energy-weighted density is W = D F D either way); the
                           batched SCF ignores it.  0 (default): the projector of
-                          rchem's eigh every iteration (rchem.rs:74-78), which small
-                          matrices (up to 128 functions) too form by products, in one
-                          launch, where F' has a gap */
+                          rchem's eigh every iteration (rchem.rs:74-78), which
+                          matrices of up to 1024 functions too form by products
+                          where F' has a gap */
   double damping;      /* a in [0, 1): each new density is mixed with the previous one,
                           D <- (1 - a) D_new + a D_old (a convergence aid for hard
                           cases; the converged density is the same stationary point);

@@ -96,6 +96,14 @@ hipError_t diis_extrapolate_launch(const double* Fs, size_t n2, const ScfDevStat
 hipError_t scf_commit_launch(double* D, const double* Dn, size_t n2, ScfDevState* st,
                              const double* coef, int steps, double tol, double damping,
                              hipStream_t s);
+hipError_t gersh_launch(const double* F, int n, double* lo, double* hi, hipStream_t s);
+size_t sp2_workspace(int n, int steps);
+hipError_t sp2_start_launch(const double* Fp, int n, const double* lo, const double* hi,
+                            double* work, int steps, hipStream_t s);
+hipError_t sp2_step_launch(double* work, int n, int nocc, int steps, int step, double* coef,
+                           hipStream_t s);
+hipError_t sp2_finish_launch(double* work, int n, int steps, int step, double* P, double* out,
+                             hipStream_t s);
 hipError_t density_small_launch(const double* F, const double* X, int ld, int nmax, const int* nb,
                                 int nocc1, const int* nocc, int count, double* D, double* flag,
                                 hipStream_t s);
@@ -2664,8 +2672,21 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
   DevBuf dflag;
   HIPC(dflag.ensure(sizeof(double) * 2 * kSmallSteps));
   if (small) HIPC(fill_launch(dflag.as<double>(), 2 * kSmallSteps, 1.0, ctx->stream));
-  DevBuf dP, dP2, dP3, dpl, dph, dpar;
-  if (opts->purify) {
+  DevBuf dP, dP2, dP3, dpl, dph, dpar, dsp2;
+  // above that, up to kSp2MaxN (where the library's products on the whole chip
+  // become the better ones), the same scheme takes one launch to a step, for
+  // either value of opts->purify; a matrix without a gap takes the eigensolver
+  constexpr int kSp2MaxN = 1024;
+  const bool sp2 = !small && n <= kSp2MaxN && opts->nocc < n;
+  if (sp2) {
+    const size_t wd = sp2_workspace(n, kPurifyMax);
+    HIPC(dsp2.ensure(wd * sizeof(double)));
+    HIPC(fill_launch(dsp2.as<double>(), wd, 0.0, ctx->stream));
+    HIPC(dP.ensure(n2 * sizeof(double)));
+    HIPC(dpl.ensure(n * sizeof(double)));
+    HIPC(dph.ensure(n * sizeof(double)));
+    HIPC(dpar.ensure((4 + 2 * kPurifyMax) * sizeof(double)));
+  } else if (opts->purify) {
     for (DevBuf* b : {&dP, &dP2, &dP3}) HIPC(b->ensure(n2 * sizeof(double)));
     HIPC(dpl.ensure(n * sizeof(double)));
     HIPC(dph.ensure(n * sizeof(double)));
@@ -2680,8 +2701,45 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
                             ctx->stream));
     return RCHEM_OK;
   };
+  // P_0 of F' (dFp) in the step kernels' workspace
+  auto sp2_start = [&]() -> int {
+    HIPC(gersh_launch(dFp.as<double>(), n, dpl.as<double>(), dph.as<double>(), ctx->stream));
+    HIPC(sp2_start_launch(dFp.as<double>(), n, dpl.as<double>(), dph.as<double>(),
+                          dsp2.as<double>(), kPurifyMax, ctx->stream));
+    return RCHEM_OK;
+  };
+  int sp2_seen = 32;  // steps the last purification of this SCF needed
   auto purify = [&](int* steps) -> int {
     *steps = 0;
+    if (sp2) {
+      // steps in bunches, one host read after each: a few more than the last
+      // time, then (no gap, or a smaller one) more until kPurifyMax
+      TRY(sp2_start());
+      double* coef = dpar.as<double>() + 4;
+      std::vector<double> c(2 * kPurifyMax);
+      int done = 0;
+      for (int upto = std::min(sp2_seen + 2, kPurifyMax); done < kPurifyMax;
+           upto = std::min(upto + 24, kPurifyMax)) {
+        for (; done < upto; ++done)
+          HIPC(sp2_step_launch(dsp2.as<double>(), n, opts->nocc, kPurifyMax, done, coef,
+                               ctx->stream));
+        HIPC(sp2_finish_launch(dsp2.as<double>(), n, kPurifyMax, done, dP.as<double>(),
+                               dpar.as<double>(), ctx->stream));
+        double ok = 0.0;
+        HIPC(hipMemcpyAsync(&ok, dpar.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        HIPC(hipMemcpyAsync(c.data(), coef, sizeof(double) * 2 * done, hipMemcpyDeviceToHost,
+                            ctx->stream));
+        HIPC(hipStreamSynchronize(ctx->stream));
+        if (ok != 0.0) {
+          int first = 0;
+          while (first < done && !(c[2 * first + 1] < kPurifyTol)) ++first;
+          *steps = sp2_seen = std::min(first + 3, kPurifyMax);
+          return RCHEM_OK;
+        }
+        if (!std::isfinite(c[2 * done - 1])) return RCHEM_OK;
+      }
+      return RCHEM_OK;
+    }
     HIPC(purify_start_launch(dFp.as<double>(), n, opts->nocc, dpl.as<double>(), dph.as<double>(),
                              dpar.as<double>(), dP.as<double>(), ctx->stream));
     int extra = -1;
@@ -2736,11 +2794,11 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
       // no gap: the purification in memory (if asked for) and the eigensolver
     }
     TRY(orthogonalise(Fm));
-    if (opts->purify) {
+    if (opts->purify || sp2) {
       int steps = 0;
       TRY(purify(&steps));
       if (steps > 0) {
-        if (psteps) *psteps = steps;
+        if (psteps && opts->purify) *psteps = steps;
         return density_from_p(Dout);
       }
     }
@@ -2847,6 +2905,19 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
         return RCHEM_OK;
       }
       TRY(orthogonalise(dFx.as<double>()));
+      if (sp2) {
+        double* coef = dpar.as<double>() + 4;
+        TRY(sp2_start());
+        for (int s = 0; s < steps; ++s)
+          HIPC(sp2_step_launch(dsp2.as<double>(), n, opts->nocc, kPurifyMax, s, coef,
+                               ctx->stream));
+        HIPC(sp2_finish_launch(dsp2.as<double>(), n, kPurifyMax, steps, dP.as<double>(),
+                               dpar.as<double>(), ctx->stream));
+        TRY(density_from_p(dDn.as<double>()));
+        HIPC(scf_commit_launch(dD.as<double>(), dDn.as<double>(), n2, st, coef, steps, kPurifyTol,
+                               opts->damping, ctx->stream));
+        return RCHEM_OK;
+      }
       HIPC(purify_start_launch(dFp.as<double>(), n, opts->nocc, dpl.as<double>(),
                                dph.as<double>(), dpar.as<double>(), dP.as<double>(), ctx->stream));
       double* coef = dpar.as<double>() + 4;

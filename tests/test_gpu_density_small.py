@@ -1,4 +1,4 @@
-"""The one-launch density (scf_density.hip) against numpy's eigenvectors."""
+"""The densities formed by products (scf_density.hip) against numpy's eigenvectors."""
 import numpy as np
 import pytest
 
@@ -22,11 +22,11 @@ def _system(n):
 
 
 @pytest.mark.parametrize("purify", [False, True])
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 48, 49, 127, 128, 129])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 48, 49, 127, 128, 129, 160, 161, 255, 257])
 def test_density_vs_eigenvectors(gpu_ctx, n, purify):
     """One plain iteration: D = the density of F(D_0), D_0 the core guess, at the
-    edges of the kernel's 16-wide tiles and of its range (128; 129 takes the
-    library's eigensolver or GEMMs).  Bar: 1e-11 -- both ways leave the
+    edges of the kernel's 16-wide tiles and of its range (128), and above it at
+    those of the step kernels' 32-wide tiles and 64-wide rows.  Bar: 1e-11 -- both ways leave the
     projector ~ n eps ||F'|| / gap off, ||F'|| ~ 5, gap ~ 0.5."""
     Z, xyz, nocc = _system(n)
     one = np.ones(n)
@@ -61,3 +61,21 @@ def test_batch_of_uneven_sizes(gpu_ctx):
         B = rb.Basis.new(Z, xyz, "STO-3G", ctx=gpu_ctx)
         one, _ = rb.scf(B, xyz, Z, nocc=sum(Z) // 2, diis=8)
         assert r.converged and one.converged and abs(r.e_total - one.e_total) < 1e-9
+
+
+def test_no_gap_takes_the_eigensolver(gpu_ctx):
+    """Three H atoms on an equilateral triangle, two orbitals occupied: the
+    second and third orbitals are degenerate, no projector of rank 2 is singled
+    out and the eigensolver picks one: Tr(D S) = 2, idempotent.  Bar 1e-10."""
+    for reps in (1, 50):  # 3 functions and 150 (far apart: 50-fold the same)
+        xyz = np.concatenate([np.array([[0, 0, 0], [2, 0, 0], [1, 3 ** 0.5, 0]]) + [0, 0, 40.0 * k]
+                              for k in range(reps)])
+        n = len(xyz)
+        one = np.ones(n)
+        B = rb.Basis.from_shells(xyz, np.zeros(n, dtype=np.int32), one.astype(np.int32),
+                                 0.5 * one, one, ctx=gpu_ctx)
+        print(f"case: no gap, {n} functions", flush=True)
+        _, D = rb.scf(B, xyz, one, nocc=2 * reps, max_iter=1, opts=default_opts())
+        S = rb.S(B)
+        assert abs(np.trace(D @ S) - 2 * reps) < 1e-10 * reps
+        assert np.abs(D @ S @ D - D).max() < 1e-10
