@@ -11,6 +11,10 @@
 namespace rchem {
 
 using EriLaunchFn = hipError_t (*)(const EriArgs&, int, hipStream_t);
+struct EriPart {
+  hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
+  size_t (*slab)(int cus) = nullptr;
+};
 
 #include "generated/eri_dispatch.inc"
 

@@ -332,6 +332,171 @@ STREAM_L = 5  # classes from this total angular momentum get a streaming kernel
 LDS_PER_LANE_BEYOND_4 = {"2120", "2210"}
 
 
+# Classes whose Fock-build kernel forms the targets in parts (eri_part.hpp):
+# parts, waves per workgroup, waves per SIMD.  More parts cost operations and
+# save registers: a primitive quartet of (dp|dp) takes 2154 vector instructions
+# in one part (386 doubles of accumulators and live values), 3228 in four (131),
+# 4171 in eight (80).  Class times of the 210-shell build, ms, with 8 parts on 8
+# waves two to a SIMD, 4 parts on 4 waves one to a SIMD, 8 parts on 4 waves two
+# workgroups to a CU: (dp|dp) 16.2, 16.5, 16.9; (dd|ds) 8.8, 8.5, 9.4; (dd|pp)
+# 8.6, 9.9, 8.7; (dd|dp) 17.9 with 16 parts, 19.5 (8 parts), 21.4 (16).  (dp|pp)
+# in 4 parts fits two workgroups to a CU: 15.5, in 8 parts 19.2.
+PART_SHAPES = {"2111": (4, 4, 2), "2121": (8, 8, 2), "2220": (8, 8, 2),
+               "2211": (8, 8, 2), "2221": (16, 8, 2), "2222": (16, 4, 1)}
+# What a part costs beside its recurrences, in vector instructions a primitive
+# quartet (the Gaussian product, the Boys function).
+PART_SETUP = 130
+
+
+def part_cost(v, ntargets):
+    """Vector instructions per primitive quartet of a part with these VRR nodes."""
+    return PART_SETUP + ntargets + sum(2 if "(" in t else 1
+                                       for ts in v.terms.values() for t in ts)
+
+
+def part_cuts(targets, nparts):
+    """Cuts of the target list into nparts runs whose largest cost is least: the
+    waves of a workgroup wait for the slowest part."""
+    def runs(limit):
+        cuts, k = [0], 0
+        while k < len(targets):
+            v, k0 = VRR(Emitter()), k
+            while k < len(targets):
+                v.node(*targets[k], 0)
+                if part_cost(v, k - k0 + 1) > limit and k > k0:
+                    break
+                k += 1
+            cuts.append(k)
+        return cuts
+
+    v = VRR(Emitter())
+    for t in targets:
+        v.node(*t, 0)
+    lo, hi = PART_SETUP, part_cost(v, len(targets))
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        if len(runs(mid)) - 1 <= nparts:
+            hi = mid
+        else:
+            lo = mid
+    cuts = runs(hi)
+    while len(cuts) - 1 < nparts:  # fewer runs sufficed: halve the longest
+        i = max(range(len(cuts) - 1), key=lambda j: cuts[j + 1] - cuts[j])
+        cuts.insert(i + 1, (cuts[i] + cuts[i + 1]) // 2)
+    return cuts
+
+
+def part_struct(la, lb, lc, ld):
+    """EriParts of one class: the VRR of each part's targets (consecutive in the
+    accumulators' order) into the part's own accumulators, the bra's horizontal
+    recurrence as a table -- (ab| = sum over k <= b of binomial(b, k)
+    AB^(b - k) [a + k 0|, at most four terms for l <= 2 -- and the ket's as
+    straight-line code on the [ab|f0) of one ab."""
+    key = f"{la}{lb}{lc}{ld}"
+    nparts, waves, minw = PART_SHAPES[key]
+    E = [t for l in range(la, la + lb + 1) for t in cart(l)]
+    F = [t for l in range(lc, lc + ld + 1) for t in cart(l)]
+    T = [(e, f) for e in E for f in F]
+    cuts = part_cuts(T, nparts)
+    out = [f"template <> struct EriParts<{la}, {lb}, {lc}, {ld}> {{",
+           f"  static constexpr int NPART = {nparts}, W = {waves}, MINW = {minw}, NF = {len(F)};",
+           "  __host__ __device__ static constexpr int begin(int p) {",
+           f"    constexpr int c[] = {{{', '.join(map(str, cuts))}}};",
+           "    return c[p];", "  }",
+           "  template <int PART>",
+           "  __device__ static __forceinline__ void vrr(const double* __restrict__ G,"
+           " double PAx, double PAy, double PAz, double WPx, double WPy, double WPz,",
+           "      double QCx, double QCy, double QCz, double WQx, double WQy, double WQz,"
+           " double oo2z, double oo2e, double oo2ze, double roz, double roe,",
+           "      double* __restrict__ acc) {",
+           "    using R = double;"]
+    for p in range(nparts):
+        em = Emitter()
+        v = VRR(em)
+        targets = {}
+        for k in range(cuts[p], cuts[p + 1]):
+            targets[v.node(*T[k], 0)] = k - cuts[p]
+        body = list(em.consts.values()) + fuse_accumulation(em.lines, v.terms, targets,
+                                                            la + lb + lc + ld)
+        out.append(f"    {'if' if p == 0 else '} else if'} constexpr (PART == {p}) {{")
+        out.extend("      " + x for x in body)
+    out += ["    }", "  }",
+            "  // bra term t of component pair ab",
+            "  __device__ static __forceinline__ PartTerm term(int ab, int t) {",
+            f"    return kPartTerms_{la}{lb}[4 * ab + t];", "  }",
+            "  // (ab|cd) of one ab from its [ab|f0), in the components' order, normalised",
+            "  __device__ static __forceinline__ void ket_hrr(const double* __restrict__ g,"
+            " double CDx, double CDy, double CDz, double* __restrict__ out) {",
+            "    (void)CDx; (void)CDy; (void)CDz;"]
+    memo = {}
+
+    def ket(c, d):
+        if (c, d) in memo:
+            return memo[(c, d)]
+        if sum(d) == 0:
+            name = f"g[{F.index(c)}]"
+        else:
+            i = next(k for k in range(3) if d[k] > 0)
+            d1 = dec(d, i)
+            t1, t2 = ket(inc(c, i), d1), ket(c, d1)
+            name = f"k{tname(c)}_{tname(d)}"
+            out.append(f"    const double {name} = {t1} + CD{AX[i]} * {t2};")
+        memo[(c, d)] = name
+        return name
+
+    k = 0
+    for c in cart(lc):
+        for d in cart(ld):
+            cn = comp_norm(c) * comp_norm(d)
+            name = ket(c, d)
+            out.append(f"    out[{k}] = {name};" if cn == 1.0 else
+                       f"    out[{k}] = {cn!r} * {name};")
+            k += 1
+    out += ["  }", "};", ""]
+    return out
+
+
+def part_terms(la, lb):
+    """The bra terms of pair class (la lb): four to a component pair, padded with zeros."""
+    E = [t for l in range(la, la + lb + 1) for t in cart(l)]
+    rows = []
+    for a in cart(la):
+        for b in cart(lb):
+            cn = comp_norm(a) * comp_norm(b)
+            terms = []
+            for kx in range(b[0] + 1):
+                for ky in range(b[1] + 1):
+                    for kz in range(b[2] + 1):
+                        c = math.comb(b[0], kx) * math.comb(b[1], ky) * math.comb(b[2], kz)
+                        e = E.index((a[0] + kx, a[1] + ky, a[2] + kz))
+                        terms.append((e, b[0] - kx, b[1] - ky, b[2] - kz, c * cn))
+            terms += [(0, 0, 0, 0, 0.0)] * (4 - len(terms))
+            rows += [f"    {{{t[0]}, {t[1]}, {t[2]}, {t[3]}, {t[4]!r}}}," for t in terms]
+    return [f"__device__ const PartTerm kPartTerms_{la}{lb}[] = {{"] + rows + ["};", ""]
+
+
+def part_tu_source(key):
+    A = ", ".join(key)
+    return "\n".join([
+        "// Generated by gen_eri.py -- do not edit.", '#include "../eri_part.hpp"', "",
+        "namespace rchem {", "",
+        f"hipError_t eri_part_launch_c{key}(const EriArgs& a, double* slab, size_t bytes, int cus,",
+        "                                    hipStream_t s) {",
+        f"  return eri_part_launch<{A}>(a, slab, bytes, cus, s);", "}",
+        f"size_t eri_part_slab_c{key}(int cus) {{ return eri_part_slab<{A}>(cus); }}", "",
+        "}  // namespace rchem", ""])
+
+
+def write_parts(out_dir):
+    parts = ["// Generated by gen_eri.py -- do not edit.", ""]
+    for bra in sorted({k[:2] for k in PART_SHAPES}):
+        parts += part_terms(int(bra[0]), int(bra[1]))
+    for key in PART_SHAPES:
+        parts += part_struct(*map(int, key))
+        write_if_changed(os.path.join(out_dir, f"eri_p_{key}.hip"), part_tu_source(key))
+    write_if_changed(os.path.join(out_dir, "eri_parts.inc"), "\n".join(parts))
+
+
 def pair_class(l1, l2):
     return l1 * (l1 + 1) // 2 + l2
 
@@ -533,6 +698,7 @@ def main():
                     fh.write(su)
     write_if_changed(os.path.join(out_dir, "eri_classes.inc"), "\n".join(parts))
     write_programs(os.path.join(out_dir, "eri_programs.inc"), lmax)
+    write_parts(out_dir)
     keys = [f"{a}{b}{c}{d}" for a, b, c, d in classes(lmax)]
     if only:
         keys = [k for k in keys if k in only]
@@ -560,6 +726,14 @@ def main():
         disp.append(f"  if (la == {k[0]} && lb == {k[1]} && lc == {k[2]} && ld == {k[3]}) "
                     f"return eri_stream_launcher_c{k}(mode);")
     disp += ["  return nullptr;", "}", ""]
+    disp += [f"hipError_t eri_part_launch_c{k}(const EriArgs&, double*, size_t, int, hipStream_t);\n"
+             f"size_t eri_part_slab_c{k}(int);" for k in PART_SHAPES]
+    disp += ["", "// Partwise Fock-build kernel of the class (exact Boys, FP64); null if none.",
+             "EriPart eri_part_launcher(int la, int lb, int lc, int ld) {"]
+    for k in PART_SHAPES:
+        disp.append(f"  if (la == {k[0]} && lb == {k[1]} && lc == {k[2]} && ld == {k[3]}) "
+                    f"return EriPart{{eri_part_launch_c{k}, eri_part_slab_c{k}}};")
+    disp += ["  return EriPart{};", "}", ""]
     write_if_changed(os.path.join(out_dir, "eri_dispatch.inc"), "\n".join(disp))
     write_if_changed(os.path.join(out_dir, "flops_per_class.json"),
                      json.dumps(flops, indent=1, sort_keys=True))

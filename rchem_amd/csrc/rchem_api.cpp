@@ -40,6 +40,13 @@ int plan_class_bits(int nclasses);
 hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s);
 EriLaunchFn eri_jk_lds_launcher(int la, int lb, int lc, int ld, int bm, int fp32, int v);
 EriStreamFn eri_stream_launcher(int la, int lb, int lc, int ld, int mode);
+// Partwise Fock-build kernel of a class: its launcher and the bytes of global
+// memory its workgroups keep a tile's accumulators in.
+struct EriPart {
+  hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
+  size_t (*slab)(int cus) = nullptr;
+};
+EriPart eri_part_launcher(int la, int lb, int lc, int ld);
 hipError_t eri_generic_launch(const EriArgs& a, const GenericProgram& p, int mode, int bm,
                               int blocks, hipStream_t s, size_t lds_limit, int shape);
 int eri_generic_shapes();
@@ -381,6 +388,8 @@ struct rchem_ctx {
 
   // LDS per workgroup of the device (hipDeviceProp_t::sharedMemPerBlock)
   size_t lds_block = 65536;
+  int cus = 256;  // compute units
+  DevBuf part_slab_d;  // the partwise kernels' accumulators beyond LDS
   // per (class, precision) launch choices of the Fock build, from the tuning
   // table (defaults where it has no entry)
   std::vector<ClassTune> tuning;
@@ -842,12 +851,17 @@ int layout_pairs(rchem_ctx* ctx, const std::vector<PairHost>& sel, double prim_e
 struct ClassKernel {
   EriLaunchFn fn = nullptr;
   EriStreamFn sfn = nullptr;  // streaming kernel (uses gp's HRR and output tables)
+  EriPart part;               // partwise kernel (kModeJK), with its workspace
+  double* slab = nullptr;
+  size_t slab_bytes = 0;
+  int cus = 0;
   const GenericProgram* gp = nullptr;
   int mode = 0, bm = 0;
   size_t lds_limit = 65536;  // the device's LDS per workgroup (wave-cooperative kernel)
   int shape = 0;             // wave-cooperative kernel's launch shape (0: chosen from the LDS)
-  bool valid() const { return fn || gp; }
+  bool valid() const { return fn || gp || part.launch; }
   hipError_t operator()(const EriArgs& a, int blocks, hipStream_t s) const {
+    if (part.launch) return blocks > 0 ? part.launch(a, slab, slab_bytes, cus, s) : hipSuccess;
     if (fn) return fn(a, blocks, s);
     if (sfn) return sfn(a, *gp, blocks, s, lds_limit);
     return eri_generic_launch(a, *gp, mode, bm, blocks, s, lds_limit, shape);
@@ -939,6 +953,17 @@ int class_kernel(rchem_ctx* ctx, int la, int lb, int lc, int ld, int mode, int b
   if (la + lb + lc + ld > kBoysMaxM) return RCHEM_OK;
   if (!ctx->force_generic) {
     const bool prefer = stream_preferred(ctx, la, lb, lc, ld);
+    // a Fock build's FP64 quartets of L >= 5, and the FP32 list of the classes
+    // without an FP32 kernel of their own
+    if (ctx->eri_stream_mode == 1 && mode == kModeJK && bm == kBoysExact && (!fp32 || prefer)) {
+      out->part = eri_part_launcher(la, lb, lc, ld);
+      if (out->part.launch) {
+        out->slab = ctx->part_slab_d.as<double>();
+        out->slab_bytes = ctx->part_slab_d.bytes;
+        out->cus = ctx->cus;
+        return RCHEM_OK;
+      }
+    }
     const EriStreamFn sfn =
         prefer && bm == kBoysExact ? eri_stream_launcher(la, lb, lc, ld, mode) : nullptr;
     if (sfn) {
@@ -1249,12 +1274,17 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   // Split tiles (PrimSplit) where a class's longest tile is longer than its
   // waves' share of the class; the tiles reserved are then counted again.
   std::vector<int> limit(nq, 0);
+  std::vector<char> partwise(nq, 0);
   bool split = false;
   for (size_t c = 0; c < nq; ++c) {
     const QClass& qc = ctx->qclasses[c];
     ClassKernel k;
     if (qc.quartets > 0)
       TRY(class_kernel(ctx, qc.la, qc.lb, qc.lc, qc.ld, kModeJK, kBoysExact, 0, &k));
+    if (k.part.launch) {
+      HIPC(ctx->part_slab_d.ensure(k.part.slab(ctx->cus)));
+      partwise[c] = 1;
+    }
     if (!k.fn) continue;  // the other engines spread a quartet over a wave
     limit[c] = split_limit(qc, iters[c]);
     if (limit[c] >= npmax[c]) limit[c] = 0;
@@ -1293,6 +1323,10 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   for (size_t c = 0; c < nq; ++c) {
     double tiles = 0.0;
     for (const double x : bra_cap[c]) tiles += x;
+    if (partwise[c]) {  // a chunk to a workgroup, one workgroup a CU
+      chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(4.0, tiles / (16.0 * ctx->cus))));
+      continue;
+    }
     chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(8.0, tiles / kMinChunks)));
   }
   // segments and passes
@@ -1762,6 +1796,10 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
                                                         " not served by this library");
           fn.shape = tn.variant;  // the class's launch shape on the wave-cooperative kernel
           a.tile_range = ranges + (prec ? 2 : 0);
+          if (fn.part.launch && ctx->lds_digestion) {
+            a.chunks = prec ? ctx->plan_chunks32.as<Chunk>() : ctx->plan_chunks64.as<Chunk>();
+            a.chunk_range = ranges + (prec ? 6 : 4);
+          }
           TRY(launch_timed(ctx, qc, prec, fn, a, std::min(tn.blocks, (cap + 3) / 4), timed_ok));
         }
       }
@@ -1873,6 +1911,7 @@ int rchem_ctx_create(int device, rchem_ctx** out) {
   auto* ctx = new rchem_ctx();
   ctx->device = device;
   ctx->lds_block = prop.sharedMemPerBlock;
+  ctx->cus = std::max(1, prop.multiProcessorCount);
   {
     // the Fock build's table, and the batched SCF's (multi-molecule bases of
     // small molecules: a bra pair has few kets, so other shapes win)
