@@ -9,7 +9,8 @@
 //              inside a bucket, so the survivors are a prefix found by binary
 //              search), split into an FP64 prefix (Q_ab Q_cd max|D| >=
 //              mixed_thresh) and an FP32 remainder; tile counts per task;
-//   3. scan:   exclusive prefix sums of the tile counts (hipCUB);
+//   3. scan:   exclusive prefix sums of the tile counts (hipCUB; FP64-only
+//              builds have one list, and no scan of the other's counts);
 //   4. expand: each task writes its tiles;
 //   5. chunks: the tiles of one (class, bra pair) unit are cut into chunks of
 //              at most the class's chunk size per precision (from the tuning
@@ -20,6 +21,8 @@
 //              memory, where the persistent ERI kernels read them.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
+
+#include <algorithm>
 
 #include "types.hpp"
 
@@ -92,6 +95,34 @@ __device__ __forceinline__ int class_of_task(const PlanArgs& a, int t) {
   return c;
 }
 
+// The kets of bra pair i in bucket slot `slot`: [lo, mid) in FP64, [mid, hi) in FP32.
+struct TaskRange {
+  int lo, mid, hi;
+};
+__device__ __forceinline__ TaskRange task_range(const PlanArgs& a, const PlanClass& pc, int i,
+                                                int slot, const int4& bk) {
+  int lo = bk.x, hi = bk.y;
+  bool all64 = false;
+  if (a.segs) {  // the bra's molecule only
+    const int mol = a.pair_mol[i];
+    const int2 sg = a.segs[static_cast<size_t>(slot) * a.nmol + mol];
+    const int state = a.mol_active ? a.mol_active[mol] : 1;
+    lo = sg.x;
+    hi = state == 0 ? sg.x : sg.y;  // a retired molecule: none
+    all64 = state == 2;             // a molecule past its precision switch: no FP32
+  }
+  if (pc.same) hi = (lo > i) ? lo : min(hi, i + 1);
+  const double qi = a.Q[i];
+  if (a.tau > 0.0) hi = (qi > 0.0) ? first_below(a.Q, lo, hi, a.tau / qi) : lo;
+  int mid = hi;
+  if (a.mixed_thresh > 0.0 && hi > lo && !all64) {
+    const double dm = *a.dmax;
+    const double need = (qi > 0.0 && dm > 0.0) ? a.mixed_thresh / (qi * dm) : HUGE_VAL;
+    mid = first_below(a.Q, lo, hi, need);
+  }
+  return TaskRange{lo, mid, hi};
+}
+
 __global__ void plan_kernel(const PlanArgs a) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = t < a.ntasks;
@@ -106,26 +137,9 @@ __global__ void plan_kernel(const PlanArgs a) {
     const PlanClass pc = a.classes[c];
     const int local = t - pc.task_begin;
     const int i = pc.bra_begin + local / pc.nbk;
-    const int4 bk = a.buckets[pc.bk_off + local % pc.nbk];
-    int lo = bk.x, hi = bk.y;
-    bool all64 = false;
-    if (a.segs) {  // the bra's molecule only
-      const int mol = a.pair_mol[i];
-      const int2 sg = a.segs[static_cast<size_t>(pc.bk_off + local % pc.nbk) * a.nmol + mol];
-      const int state = a.mol_active ? a.mol_active[mol] : 1;
-      lo = sg.x;
-      hi = state == 0 ? sg.x : sg.y;  // a retired molecule: none
-      all64 = state == 2;             // a molecule past its precision switch: no FP32
-    }
-    if (pc.same) hi = (lo > i) ? lo : min(hi, i + 1);
-    const double qi = a.Q[i];
-    if (a.tau > 0.0) hi = (qi > 0.0) ? first_below(a.Q, lo, hi, a.tau / qi) : lo;
-    int mid = hi;
-    if (a.mixed_thresh > 0.0 && hi > lo && !all64) {
-      const double dm = *a.dmax;
-      const double need = (qi > 0.0 && dm > 0.0) ? a.mixed_thresh / (qi * dm) : HUGE_VAL;
-      mid = first_below(a.Q, lo, hi, need);
-    }
+    const int slot = pc.bk_off + local % pc.nbk;
+    const int4 bk = a.buckets[slot];
+    const auto [lo, mid, hi] = task_range(a, pc, i, slot, bk);
     a.lo[t] = lo;
     a.mid[t] = mid;
     a.hi[t] = hi;
@@ -179,6 +193,7 @@ __global__ void expand_kernel(const PlanArgs a, const int* __restrict__ off64,
   for (int k = lo; k < mid; k += 64)
     for (int p = 0; p < parts && o < cap; ++p, ++o)
       tiles64[o] = Tile{i, k, min(64, mid - k), sp.pad(p)};
+  if (!off32) return;
   o = off32[t];
   for (int k = mid; k < hi; k += 64)
     for (int p = 0; p < parts && o < cap; ++p, ++o)
@@ -216,7 +231,7 @@ __global__ void chunk_count_kernel(const PlanArgs a, const int* __restrict__ off
   unit_tasks(a, u, &c, &bra, &t0, &t1);
   const int ch64 = a.classes[c].chunk64, ch32 = a.classes[c].chunk32;
   chc64[u] = (off64[t1] - off64[t0] + ch64 - 1) / ch64;
-  chc32[u] = (off32[t1] - off32[t0] + ch32 - 1) / ch32;
+  if (off32) chc32[u] = (off32[t1] - off32[t0] + ch32 - 1) / ch32;
 }
 
 // cap bounds the tile offsets (tile buffers), ccap the chunk records written
@@ -247,7 +262,7 @@ __global__ void chunk_expand_kernel(const PlanArgs a, const int* __restrict__ of
       if (keys64) keys64[o] = khigh | ((order & 1) ? static_cast<unsigned>(tiles64[k].ket0 >> 6) : 0u);
     }
   }
-  {
+  if (off32) {
     const int ch = a.classes[c].chunk32;
     const int tb = min(off32[t0], cap), te = min(off32[t1], cap);
     int o = choff32[u];
@@ -256,6 +271,136 @@ __global__ void chunk_expand_kernel(const PlanArgs a, const int* __restrict__ of
       if (keys32) keys32[o] = khigh | ((order & 2) ? static_cast<unsigned>(tiles32[k].ket0 >> 6) : 0u);
     }
   }
+}
+
+// The whole plan of a pass in one launch, for passes of little work: 16 lanes to a
+// unit, each class's tiles and chunks in a range of their own (PlanClass::base;
+// the capacities are upper bounds), handed out to the units by counters -- the
+// range ends in `ranges`, which begin_kernel has set to the bases -- so a
+// class's units come in any order.  One block's units of a class take their
+// places with one atomic.
+constexpr int kDirectLanes = 16;
+
+__global__ __launch_bounds__(256) void plan_direct_kernel(const PlanArgs a,
+                                                          Tile* __restrict__ tiles64,
+                                                          Tile* __restrict__ tiles32,
+                                                          Chunk* __restrict__ chunks64,
+                                                          Chunk* __restrict__ chunks32, int cap,
+                                                          int* __restrict__ ranges) {
+  constexpr int G = 256 / kDirectLanes;
+  __shared__ int sc[G], sn[4][G], sbase[4][G];
+  __shared__ double sq[4][G];
+  const int g = threadIdx.x / kDirectLanes, l = threadIdx.x % kDirectLanes;
+  const int u = blockIdx.x * G + g;
+  const bool valid = u < a.nunits;
+  int c = -1, bra = 0, t0 = 0, t1 = 0;
+  PlanClass pc{};
+  if (valid) {
+    unit_tasks(a, u, &c, &bra, &t0, &t1);
+    pc = a.classes[c];
+  }
+  const int np = valid ? a.pairs[bra].np : 0;
+  int n[2] = {0, 0};  // tiles, FP64 and FP32
+  double q[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int t = t0 + l; t < t1; t += kDirectLanes) {
+    const int slot = pc.bk_off + t - t0;
+    const int4 bk = a.buckets[slot];
+    const auto [lo, mid, hi] = task_range(a, pc, bra, slot, bk);
+    a.lo[t] = lo;
+    a.mid[t] = mid;
+    a.hi[t] = hi;
+    const int parts = PrimSplit(np, bk.z, pc.limit).parts();
+    n[0] += ((mid - lo + 63) >> 6) * parts;
+    n[1] += ((hi - mid + 63) >> 6) * parts;
+    const double npp = static_cast<double>(np) * bk.z;
+    q[0] += mid - lo;
+    q[1] += hi - mid;
+    q[2] += (mid - lo) * npp;
+    q[3] += (hi - mid) * npp;
+  }
+  for (int off = kDirectLanes / 2; off > 0; off >>= 1) {
+    for (int p = 0; p < 2; ++p) n[p] += __shfl_xor(n[p], off, kDirectLanes);
+    for (int k = 0; k < 4; ++k) q[k] += __shfl_xor(q[k], off, kDirectLanes);
+  }
+  const int ch[2] = {pc.chunk64, pc.chunk32};
+  if (l == 0) {
+    sc[g] = c;
+    for (int p = 0; p < 2; ++p) {
+      sn[p][g] = n[p];
+      sn[2 + p][g] = valid ? (n[p] + ch[p] - 1) / ch[p] : 0;
+    }
+    for (int k = 0; k < 4; ++k) sq[k][g] = q[k];
+  }
+  __syncthreads();
+  int first = g, before[4] = {0, 0, 0, 0};
+  for (int h = g - 1; h >= 0 && sc[h] == c; --h) {
+    first = h;
+    for (int k = 0; k < 4; ++k) before[k] += sn[k][h];
+  }
+  if (valid && l < 4 && first == g) {  // lane k: list k of the block's units of the class
+    int total = 0;
+    double s = 0.0;
+    for (int h = g; h < G && sc[h] == c; ++h) {
+      total += sn[l][h];
+      s += sq[l][h];
+    }
+    sbase[l][g] = total > 0 ? atomicAdd(&ranges[8 * c + 2 * l + 1], total) : 0;
+    if (s > 0.0)
+      unsafeAtomicAdd(a.stats + static_cast<size_t>(blockIdx.x & (kPlanStatsReplicas - 1)) *
+                                    a.stats_stride + 4 * c + l,
+                      s);
+  }
+  __syncthreads();
+  if (!valid) return;
+  for (int p = 0; p < 2; ++p) {
+    if (n[p] == 0) continue;
+    Tile* const tiles = p ? tiles32 : tiles64;
+    Chunk* const chunks = p ? chunks32 : chunks64;
+    const int ob = sbase[p][first] + before[p];
+    const int cb = sbase[2 + p][first] + before[2 + p], nch = (n[p] + ch[p] - 1) / ch[p];
+    for (int x = l; x < nch; x += kDirectLanes)
+      if (cb + x < cap)
+        chunks[cb + x] = Chunk{bra, ob + x * ch[p], min(ob + (x + 1) * ch[p], ob + n[p]), 0};
+    int o = ob;
+    for (int t = t0; t < t1; t += kDirectLanes) {
+      int from = 0, to = 0, knp = 0;  // of the lane's own task
+      if (t + l < t1) {
+        from = p ? a.mid[t + l] : a.lo[t + l];
+        to = p ? a.hi[t + l] : a.mid[t + l];
+        knp = a.buckets[pc.bk_off + t + l - t0].z;
+      }
+      for (int j = 0; j < min(kDirectLanes, t1 - t); ++j) {
+        const int kb = __shfl(from, j, kDirectLanes), ke = __shfl(to, j, kDirectLanes);
+        const PrimSplit sp(np, __shfl(knp, j, kDirectLanes), pc.limit);
+        const int parts = sp.parts(), m = ((ke - kb + 63) >> 6) * parts;
+        for (int x = l; x < m; x += kDirectLanes) {
+          const int k = kb + 64 * (x / parts);
+          if (o + x < cap) tiles[o + x] = Tile{bra, k, min(64, ke - k), sp.pad(x % parts)};
+        }
+        o += m;
+      }
+    }
+  }
+}
+
+// Clears a build's accumulators (n2 = 0: J and K are cleared elsewhere) and sets
+// every class's tile and chunk ranges to its base, empty.
+__global__ void begin_kernel(double* __restrict__ J, double* __restrict__ K, size_t n2,
+                             double* __restrict__ stats, size_t nstats, double* __restrict__ jp,
+                             size_t njp, double* __restrict__ dmax,
+                             const PlanClass* __restrict__ classes, int nclasses,
+                             int* __restrict__ ranges) {
+  const size_t i0 = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
+  const size_t step = static_cast<size_t>(gridDim.x) * blockDim.x;
+  for (size_t i = i0; i < n2; i += step) {
+    J[i] = 0.0;
+    K[i] = 0.0;
+  }
+  for (size_t i = i0; i < njp; i += step) jp[i] = 0.0;
+  for (size_t i = i0; i < nstats; i += step) stats[i] = 0.0;
+  if (i0 == 0) *dmax = 0.0;
+  for (size_t i = i0; i < 8 * static_cast<size_t>(nclasses); i += step)
+    ranges[i] = classes[i / 8].base;
 }
 
 // keys[i] = all ones for i in [total, n): the entries past the chunk count
@@ -280,12 +425,12 @@ __global__ void ranges_kernel(const PlanArgs a, const int* __restrict__ off64,
   const int ue = (c + 1 < a.nclasses) ? a.classes[c + 1].unit_begin : a.nunits;
   ranges[8 * c + 0] = min(off64[tb], cap);
   ranges[8 * c + 1] = min(off64[te], cap);
-  ranges[8 * c + 2] = min(off32[tb], cap);
-  ranges[8 * c + 3] = min(off32[te], cap);
+  ranges[8 * c + 2] = off32 ? min(off32[tb], cap) : 0;
+  ranges[8 * c + 3] = off32 ? min(off32[te], cap) : 0;
   ranges[8 * c + 4] = min(choff64[ub], ccap);
   ranges[8 * c + 5] = min(choff64[ue], ccap);
-  ranges[8 * c + 6] = min(choff32[ub], ccap);
-  ranges[8 * c + 7] = min(choff32[ue], ccap);
+  ranges[8 * c + 6] = off32 ? min(choff32[ub], ccap) : 0;
+  ranges[8 * c + 7] = off32 ? min(choff32[ue], ccap) : 0;
 }
 
 hipError_t dmax_launch(const double* D, size_t n2, unsigned long long* out, hipStream_t s) {
@@ -332,7 +477,24 @@ size_t plan_scan_bytes(int n) {
   return bytes;
 }
 
+hipError_t begin_launch(double* J, double* K, size_t n2, double* stats, size_t nstats, double* jp,
+                        size_t njp, double* dmax, const PlanClass* classes, int nclasses,
+                        int* ranges, hipStream_t s) {
+  const size_t most = std::max({n2, nstats, njp, static_cast<size_t>(8) * nclasses});
+  const unsigned blocks = static_cast<unsigned>(std::min<size_t>(2048, (most + 255) / 256));
+  hipLaunchKernelGGL(begin_kernel, dim3(std::max(1u, blocks)), dim3(256), 0, s, J, K, n2, stats,
+                     nstats, jp, njp, dmax, classes, nclasses, ranges);
+  return hipGetLastError();
+}
+
 hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s) {
+  if (b.direct) {
+    if (a.nunits <= 0) return hipSuccess;
+    constexpr int units = 256 / kDirectLanes;
+    hipLaunchKernelGGL(plan_direct_kernel, dim3((a.nunits + units - 1) / units), dim3(256), 0, s,
+                       a, b.tiles64, b.tiles32, b.chunks64, b.chunks32, b.cap, b.ranges);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(plan_kernel, dim3(static_cast<unsigned>((a.ntasks + 1 + 255) / 256)),
                      dim3(256), 0, s, a);
   hipError_t e = hipGetLastError();
@@ -340,25 +502,30 @@ hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s) {
   size_t sb = b.scan_bytes;
   e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, a.cnt64, b.off64, a.ntasks + 1, s);
   if (e != hipSuccess) return e;
-  sb = b.scan_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, a.cnt32, b.off32, a.ntasks + 1, s);
-  if (e != hipSuccess) return e;
+  const int* off32 = a.mixed_thresh > 0.0 ? b.off32 : nullptr;  // null: no FP32 list
+  if (off32) {
+    sb = b.scan_bytes;
+    e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, a.cnt32, b.off32, a.ntasks + 1, s);
+    if (e != hipSuccess) return e;
+  }
   if (a.ntasks > 0) {
     hipLaunchKernelGGL(expand_kernel, dim3(static_cast<unsigned>((a.ntasks + 255) / 256)),
-                       dim3(256), 0, s, a, b.off64, b.off32, b.tiles64, b.tiles32, b.cap);
+                       dim3(256), 0, s, a, b.off64, off32, b.tiles64, b.tiles32, b.cap);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(chunk_count_kernel, dim3(static_cast<unsigned>((a.nunits + 1 + 255) / 256)),
-                     dim3(256), 0, s, a, b.off64, b.off32, b.chc64, b.chc32);
+                     dim3(256), 0, s, a, b.off64, off32, b.chc64, b.chc32);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   sb = b.scan_bytes;
   e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, b.chc64, b.choff64, a.nunits + 1, s);
   if (e != hipSuccess) return e;
-  sb = b.scan_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, b.chc32, b.choff32, a.nunits + 1, s);
-  if (e != hipSuccess) return e;
+  if (off32) {
+    sb = b.scan_bytes;
+    e = hipcub::DeviceScan::ExclusiveSum(b.scan_tmp, sb, b.chc32, b.choff32, a.nunits + 1, s);
+    if (e != hipSuccess) return e;
+  }
   const bool sorting = b.key_bits > 0 && b.ccap > 0;
   const bool sort64 = sorting && (b.sort_mask & 1);
   // FP64-only builds have no FP32 chunks
@@ -371,7 +538,7 @@ hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s) {
   unsigned* k32 = sort32 ? b.keys_raw + b.ccap : nullptr;
   if (a.nunits > 0) {
     hipLaunchKernelGGL(chunk_expand_kernel, dim3(static_cast<unsigned>((a.nunits + 255) / 256)),
-                       dim3(256), 0, s, a, b.off64, b.off32, b.choff64, b.choff32, out64, out32,
+                       dim3(256), 0, s, a, b.off64, off32, b.choff64, b.choff32, out64, out32,
                        b.cap, ccap, b.tiles64, b.tiles32, k64, k32,
                        b.key_bits - plan_class_bits(a.nclasses));
     e = hipGetLastError();
@@ -391,7 +558,7 @@ hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s) {
                                            p ? b.chunks32 : b.chunks64, b.ccap, 0, b.key_bits, s);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(ranges_kernel, dim3(1), dim3(64), 0, s, a, b.off64, b.off32, b.choff64,
+  hipLaunchKernelGGL(ranges_kernel, dim3(1), dim3(64), 0, s, a, b.off64, off32, b.choff64,
                      b.choff32, b.ranges, b.cap, ccap);
   return hipGetLastError();
 }

@@ -37,6 +37,9 @@ hipError_t dmax_blocks_launch(const double* D, size_t n, const int* f0, const in
 size_t plan_scan_bytes(int ntasks);
 size_t plan_sort_bytes(int n);
 int plan_class_bits(int nclasses);
+hipError_t begin_launch(double* J, double* K, size_t n2, double* stats, size_t nstats, double* jp,
+                        size_t njp, double* dmax, const PlanClass* classes, int nclasses,
+                        int* ranges, hipStream_t s);
 hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s);
 EriLaunchFn eri_jk_lds_launcher(int la, int lb, int lc, int ld, int bm, int fp32, int v);
 EriStreamFn eri_stream_launcher(int la, int lb, int lc, int ld, int mode);
@@ -1220,6 +1223,14 @@ constexpr double kMinChunks = 1024.0;
 
 // Device-planner tables for threshold tau: classes, buckets, capacities and
 // the FP64 statistics (exact for all-FP64 builds).
+// Passes of at most this many tiles are planned in one launch, a class's units
+// in any order.  The scans and sorts of the ordered plan are some ten launches
+// (FP64 water STO-3G 0.185 -> 0.155 ms, its 27-iteration SCF 7.2 -> 6.5 ms), but
+// their order spreads the work evenly over the workgroups that take it round
+// robin: at 99 000 tiles ((H2O)_8) the two are level, (10|00) 0.13 against
+// 0.17 ms, at 176 000 the ordered plan is ahead ((H2O)_12 gradient with its SCF
+// 53.2 against 54.9 ms), at 3.2 million by 17 % ((H2O)_64).
+constexpr int kDirectPlanTiles = 65536;
 constexpr double kPassTiles = 67108864.0;  // 2^26 tiles (1 GiB per tile list) per pass
 
 int prepare_plan(rchem_ctx* ctx, double tau) {
@@ -1354,6 +1365,7 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
     const ClassTune t64 = tune_for(ctx, qc.la, qc.lb, qc.lc, qc.ld, 0);
     const ClassTune t32 = tune_for(ctx, qc.la, qc.lb, qc.lc, qc.ld, 1);
     pc.limit = limit[c];
+    pc.base = static_cast<int>(pass_cap);
     pc.chunk64 = std::min(t64.chunk_tiles, chunk_most[c]);
     pc.chunk32 = std::min(t32.chunk_tiles, chunk_most[c]);
     pc.order = (ket_order_of(ctx, t64) ? 1 : 0) | (ket_order_of(ctx, t32) ? 2 : 0);
@@ -1671,18 +1683,16 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
   ctx->last_stats_dev = bf.stats;
   const bool timed_ok = ext == nullptr;
   const bool blocks = ctx->nmol > 1 && ctx->mol_nmax > 0;  // block-diagonal J and K
-  if (blocks) {
+  if (blocks)
     HIPC(fill_blocks_launch(bf.Jh, bf.Kh, ctx->nbf, ctx->mol_f0_d.as<int>(), ctx->mol_nb_d.as<int>(),
                             ctx->nmol, ctx->mol_nmax, ctx->stream));
-  } else {
-    HIPC(fill_launch(bf.Jh, n2, 0.0, ctx->stream));
-    HIPC(fill_launch(bf.Kh, n2, 0.0, ctx->stream));
-  }
   const int nc = static_cast<int>(ctx->pclasses.size());
-  HIPC(fill_launch(bf.stats, 4 * kPlanStatsReplicas * static_cast<size_t>(std::max(nc, 1)), 0.0,
-                   ctx->stream));
+  HIPC(begin_launch(bf.Jh, bf.Kh, blocks ? 0 : n2, bf.stats,
+                    4 * kPlanStatsReplicas * static_cast<size_t>(std::max(nc, 1)), bf.jp,
+                    std::max<size_t>(ctx->jp_size, 1), bf.dmax,
+                    ctx->plan_classes_d.as<PlanClass>(), nc, ctx->plan_ranges.as<int>(),
+                    ctx->stream));
   if (mixed) {
-    HIPC(fill_launch(bf.dmax, 1, 0.0, ctx->stream));
     if (ctx->nmol > 1 && ctx->mol_nmax > 0)  // a multi-molecule basis: its diagonal blocks
       HIPC(dmax_blocks_launch(dD, static_cast<size_t>(ctx->nbf), ctx->mol_f0_d.as<int>(),
                               ctx->mol_nb_d.as<int>(), ctx->nmol, ctx->mol_nmax,
@@ -1690,7 +1700,6 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
     else
       HIPC(dmax_launch(dD, n2, reinterpret_cast<unsigned long long*>(bf.dmax), ctx->stream));
   }
-  HIPC(fill_launch(bf.jp, std::max<size_t>(ctx->jp_size, 1), 0.0, ctx->stream));
   // the pairs' density blocks in the Jp layout, for the LDS kernels' Coulomb sums
   HIPC(dpair_gather_launch(ctx->pairs_d.as<PairRec>(), dD, ctx->jp_cls_d.as<JpClass>(),
                            ctx->jp_ncomp_d.as<int>(), kNumPairClasses,
@@ -1733,6 +1742,7 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
     pb.chunks64 = ctx->plan_chunks64.as<Chunk>();
     pb.chunks32 = ctx->plan_chunks32.as<Chunk>();
     pb.cap = ps.cap;
+    pb.direct = ps.cap <= kDirectPlanTiles;
     pb.ranges = ctx->plan_ranges.as<int>() + 8 * static_cast<size_t>(ps.seg_begin);
     pb.scan_tmp = ctx->plan_scan_tmp.p;
     pb.scan_bytes = ctx->plan_scan_bytes;

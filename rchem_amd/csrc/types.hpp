@@ -231,6 +231,8 @@ struct PlanClass {
   int chunk64, chunk32;    // tiles per LDS-digestion chunk, FP64 and FP32 lists
   int order;               // bit 0 / 1: FP64 / FP32 chunks ordered by first ket pair
   int limit;               // PrimSplit's limit
+  int base;                // first entry of the class in the tile and chunk lists of a pass
+                           // that is planned without scans (its capacity follows)
 };
 
 struct PlanArgs {
@@ -275,6 +277,7 @@ struct PlanBuffers {
   Chunk* chunks32;
   int cap;
   int* ranges;       // 8 per class
+  bool direct;       // plan in one launch, a class's units in any order
   void* scan_tmp;
   size_t scan_bytes;
   // chunk order by ket window (key_bits > 0): the chunks are written unsorted
