@@ -143,8 +143,11 @@ __global__ __launch_bounds__(THREADS, MINW) void eri_part_kernel(
   for (int k = tid; k < NC * ND * 64; k += THREADS) jq[k] = 0.0;
   const int begin = ROWS ? a.chunk_range[0] : a.tile_range ? a.tile_range[0] : 0;
   const int end = ROWS ? a.chunk_range[1] : a.tile_range ? a.tile_range[1] : a.ntiles;
-  for (int u = begin + static_cast<int>(blockIdx.x); u < end;
-       u += static_cast<int>(gridDim.x)) {  // block-uniform
+  __shared__ int s_next[2];  // by turns: a chunk may have no barrier but its last
+  int turn = 0;
+  for (int u = begin + static_cast<int>(blockIdx.x); u < end;) {  // block-uniform
+    int next = 0;
+    if (ROWS && tid == 0) next = atomicAdd(a.next, 1);  // awaited at the chunk's end
     const Chunk ch = ROWS ? chunks[u] : Chunk{tiles[u].bra, u, u + 1, 0};
     const int kc0 = ROWS && a.pair_kc0 ? a.pair_kc0[ch.bra] : 0;
     const PairRec bp = pairs[ch.bra];
@@ -297,7 +300,11 @@ __global__ __launch_bounds__(THREADS, MINW) void eri_part_kernel(
         }
       }
     }
+    if (ROWS && tid == 0) s_next[turn] = next;
     __syncthreads();
+    u = ROWS ? begin + static_cast<int>(gridDim.x) + __builtin_amdgcn_readfirstlane(s_next[turn])
+             : u + static_cast<int>(gridDim.x);
+    turn ^= 1;
   }
 }
 

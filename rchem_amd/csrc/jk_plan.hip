@@ -383,13 +383,13 @@ __global__ __launch_bounds__(256) void plan_direct_kernel(const PlanArgs a,
   }
 }
 
-// Clears a build's accumulators (n2 = 0: J and K are cleared elsewhere) and sets
-// every class's tile and chunk ranges to its base, empty.
+// Clears a build's accumulators (n2 = 0: J and K are cleared elsewhere) and its
+// chunk counters, and sets every class's tile and chunk ranges to its base, empty.
 __global__ void begin_kernel(double* __restrict__ J, double* __restrict__ K, size_t n2,
                              double* __restrict__ stats, size_t nstats, double* __restrict__ jp,
                              size_t njp, double* __restrict__ dmax,
                              const PlanClass* __restrict__ classes, int nclasses,
-                             int* __restrict__ ranges) {
+                             int* __restrict__ ranges, int* __restrict__ next) {
   const size_t i0 = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
   const size_t step = static_cast<size_t>(gridDim.x) * blockDim.x;
   for (size_t i = i0; i < n2; i += step) {
@@ -401,6 +401,7 @@ __global__ void begin_kernel(double* __restrict__ J, double* __restrict__ K, siz
   if (i0 == 0) *dmax = 0.0;
   for (size_t i = i0; i < 8 * static_cast<size_t>(nclasses); i += step)
     ranges[i] = classes[i / 8].base;
+  for (size_t i = i0; i < 2 * static_cast<size_t>(nclasses); i += step) next[i] = 0;
 }
 
 // keys[i] = all ones for i in [total, n): the entries past the chunk count
@@ -479,11 +480,11 @@ size_t plan_scan_bytes(int n) {
 
 hipError_t begin_launch(double* J, double* K, size_t n2, double* stats, size_t nstats, double* jp,
                         size_t njp, double* dmax, const PlanClass* classes, int nclasses,
-                        int* ranges, hipStream_t s) {
+                        int* ranges, int* next, hipStream_t s) {
   const size_t most = std::max({n2, nstats, njp, static_cast<size_t>(8) * nclasses});
   const unsigned blocks = static_cast<unsigned>(std::min<size_t>(2048, (most + 255) / 256));
   hipLaunchKernelGGL(begin_kernel, dim3(std::max(1u, blocks)), dim3(256), 0, s, J, K, n2, stats,
-                     nstats, jp, njp, dmax, classes, nclasses, ranges);
+                     nstats, jp, njp, dmax, classes, nclasses, ranges, next);
   return hipGetLastError();
 }
 

@@ -39,7 +39,7 @@ size_t plan_sort_bytes(int n);
 int plan_class_bits(int nclasses);
 hipError_t begin_launch(double* J, double* K, size_t n2, double* stats, size_t nstats, double* jp,
                         size_t njp, double* dmax, const PlanClass* classes, int nclasses,
-                        int* ranges, hipStream_t s);
+                        int* ranges, int* next, hipStream_t s);
 hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s);
 EriLaunchFn eri_jk_lds_launcher(int la, int lb, int lc, int ld, int bm, int fp32, int v);
 EriStreamFn eri_stream_launcher(int la, int lb, int lc, int ld, int mode);
@@ -372,6 +372,7 @@ struct rchem_ctx {
   int chunk_order_env = -1;
   int plan_key_bits = 0, plan_ccap = 0;
   size_t plan_sort_bytes = 0;
+  DevBuf plan_next;
   DevBuf plan_chunks_raw, plan_keys_raw, plan_keys_sorted, plan_sort_tmp;
   // pair-indexed Coulomb accumulators
   std::vector<JpClass> jp_cls;
@@ -1467,6 +1468,7 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   HIPC(ctx->plan_tiles64.ensure(sizeof(Tile) * static_cast<size_t>(ctx->plan_cap)));
   HIPC(ctx->plan_tiles32.ensure(sizeof(Tile) * static_cast<size_t>(ctx->plan_cap)));
   HIPC(ctx->plan_ranges.ensure(sizeof(int) * 8 * std::max<size_t>(ctx->pclasses.size(), 1)));
+  HIPC(ctx->plan_next.ensure(sizeof(int) * 2 * std::max<size_t>(ctx->pclasses.size(), 1)));
   HIPC(ctx->plan_stats.ensure(sizeof(double) * 4 * kPlanStatsReplicas *
                               std::max<size_t>(ctx->pclasses.size(), 1)));
   HIPC(ctx->plan_dmax.ensure(sizeof(double)));
@@ -1691,7 +1693,7 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
                     4 * kPlanStatsReplicas * static_cast<size_t>(std::max(nc, 1)), bf.jp,
                     std::max<size_t>(ctx->jp_size, 1), bf.dmax,
                     ctx->plan_classes_d.as<PlanClass>(), nc, ctx->plan_ranges.as<int>(),
-                    ctx->stream));
+                    ctx->plan_next.as<int>(), ctx->stream));
   if (mixed) {
     if (ctx->nmol > 1 && ctx->mol_nmax > 0)  // a multi-molecule basis: its diagonal blocks
       HIPC(dmax_blocks_launch(dD, static_cast<size_t>(ctx->nbf), ctx->mol_f0_d.as<int>(),
@@ -1809,6 +1811,7 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
           if (fn.part.launch && ctx->lds_digestion) {
             a.chunks = prec ? ctx->plan_chunks32.as<Chunk>() : ctx->plan_chunks64.as<Chunk>();
             a.chunk_range = ranges + (prec ? 6 : 4);
+            a.next = ctx->plan_next.as<int>() + 2 * sg + prec;
           }
           TRY(launch_timed(ctx, qc, prec, fn, a, std::min(tn.blocks, (cap + 3) / 4), timed_ok));
         }

@@ -162,6 +162,7 @@ struct EriArgs {
   // LDS digestion (chunked launches): K rows of the bra in LDS, J by pair
   const Chunk* chunks;
   const int* chunk_range;  // [begin, end) in chunks, device memory
+  int* next;               // chunks handed out beyond the first of each workgroup
   double* Jp;
   JpClass jp_bra, jp_ket;
   const double* Dp;  // the density blocks of the pairs, in Jp's layout (null: gather from D)
