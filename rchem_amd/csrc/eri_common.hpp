@@ -124,8 +124,14 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
   constexpr int L = C::L;
   constexpr bool KP = MODE == kModeJK;
   static_assert(BM == kBoysExact || sizeof(R) == 8, "compat Boys is FP64 only");
-  ti.active = lane < t.count;
-  const int lane_off = ti.active ? lane : 0;  // an idle lane repeats the first
+  // kModeTensor: 1 << sh lanes to a quartet, each with every (1 << sh)-th ket
+  // primitive pair
+  constexpr bool SPLIT = MODE == kModeTensor;
+  const int sh = SPLIT ? t.pad : 0;
+  const int part = SPLIT ? lane & ((1 << sh) - 1) : 0;
+  const int q = SPLIT ? lane >> sh : lane;
+  ti.active = q < t.count;
+  const int lane_off = ti.active ? q : 0;  // an idle lane repeats the first
   ti.kidx = t.ket0 + lane_off;
   if constexpr (!KP) {
     ti.bidx = (MODE == kModeDiag) ? ti.kidx : t.bra;
@@ -190,13 +196,23 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
     row = 0;
     row_off = kp.p0;
   }
-  P nxt = load_ket_prim<R, KP>(src.ket, prim, row, row_off);
-  for (int j = 0; j < knp; ++j) {
+  // the lane's j-th ket record; beyond its last it takes the first, with no weight
+  auto in_part = [&](int j) { return !SPLIT || (j << sh) + part < knp; };
+  auto ket_prim = [&](int j) __attribute__((always_inline)) {
+    if constexpr (SPLIT)
+      return load_ket_prim<R, KP>(src.ket, prim, 0,
+                                  row_off + (in_part(j) ? ((j << sh) + part) * kps : 0));
+    else
+      return load_ket_prim<R, KP>(src.ket, prim, row + j * kps, row_off);
+  };
+  const int jn = SPLIT ? (knp + (1 << sh) - 1) >> sh : knp;
+  P nxt = ket_prim(0);
+  for (int j = 0; j < jn; ++j) {
     // with PF the next record is in flight during this iteration's work;
     // without, the load is issued here and other waves cover its latency
-    const P pk = PF ? nxt : load_ket_prim<R, KP>(src.ket, prim, row + j * kps, row_off);
-    if (PF && j + 1 < knp) nxt = load_ket_prim<R, KP>(src.ket, prim, row + (j + 1) * kps, row_off);
-    const R zk = R(pk.zeta), kk = R(pk.kab), oo2e = R(pk.oo2z);
+    const P pk = PF ? nxt : ket_prim(j);
+    if (PF && j + 1 < jn) nxt = ket_prim(j + 1);
+    const R zk = R(pk.zeta), kk = in_part(j) ? R(pk.kab) : R(0), oo2e = R(pk.oo2z);
     const R QCx = R(pk.pax), QCy = R(pk.pay), QCz = R(pk.paz);
     const R QAx = QCx - ACx, QAy = QCy - ACy, QAz = QCz - ACz;
     // one bra primitive pair into the accumulators
@@ -248,6 +264,12 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
     }
   }
 
+  if constexpr (SPLIT) {
+    for (int off = (1 << sh) >> 1; off > 0; off >>= 1) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < C::NACC; ++i) acc[i] += __shfl_xor(acc[i], off, 64);
+    }
+  }
   R outr[C::NOUT];
   C::template hrr<R>(acc, R(bp.AB[0]), R(bp.AB[1]), R(bp.AB[2]), R(kp.AB[0]), R(kp.AB[1]),
                      R(kp.AB[2]), outr);
@@ -461,26 +483,37 @@ __device__ __forceinline__ void eri_tile(const EriArgs& a, const TileSrc& src, c
     }
   } else if constexpr (MODE == kModeTensor) {
     if (ti.active) {
+      // the eight index orders, shared by the quartet's lanes
+      for (int w = lane & ((1 << t.pad) - 1); w < 8; w += 1 << t.pad) {
+        size_t sp = n * n * n, sq = n * n, sr = n, ss = 1;  // strides of a, b, c, d
+        if (w & 1) {
+          const size_t x = sp;
+          sp = sq;
+          sq = x;
+        }
+        if (w & 2) {
+          sr = 1;
+          ss = n;
+        }
+        if (w & 4) {
+          size_t x = sp;
+          sp = sr;
+          sr = x;
+          x = sq;
+          sq = ss;
+          ss = x;
+        }
+        double* const I = a.out + fa * sp + fb * sq + fc * sr + fd * ss;
 #pragma unroll
-      for (int ia = 0; ia < NA; ++ia)
+        for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
-        for (int ib = 0; ib < NB; ++ib)
+          for (int ib = 0; ib < NB; ++ib)
 #pragma unroll
-          for (int ic = 0; ic < NC; ++ic)
+            for (int ic = 0; ic < NC; ++ic)
 #pragma unroll
-            for (int id = 0; id < ND; ++id) {
-              const double v = out[((ia * NB + ib) * NC + ic) * ND + id];
-              const size_t p = fa + ia, q = fb + ib, r = fc + ic, s = fd + id;
-              double* I = a.out;
-              I[((p * n + q) * n + r) * n + s] = v;
-              I[((q * n + p) * n + r) * n + s] = v;
-              I[((p * n + q) * n + s) * n + r] = v;
-              I[((q * n + p) * n + s) * n + r] = v;
-              I[((r * n + s) * n + p) * n + q] = v;
-              I[((s * n + r) * n + p) * n + q] = v;
-              I[((r * n + s) * n + q) * n + p] = v;
-              I[((s * n + r) * n + q) * n + p] = v;
-            }
+              for (int id = 0; id < ND; ++id)
+                I[ia * sp + ib * sq + ic * sr + id * ss] = out[((ia * NB + ib) * NC + ic) * ND + id];
+      }
     }
   } else {
     const double s = symmetry_weight(ti);

@@ -1168,6 +1168,13 @@ double per_prim_flops(const QClass& qc, int* hrr) {
   return fv + 68.0 + 4.0 * (qc.la + qc.lb + qc.lc + qc.ld);
 }
 
+// Lanes to a quartet of the tensor kernels: at most 8, and no more than give the
+// class 8 waves to a SIMD.  A lane's chain of
+// primitive quartets was the time of a small tensor's kernels: (H2O)_3 6-31G
+// (ss|ss) 0.289 -> 0.080 ms, all classes 0.89 -> 0.23, the call 2.35 -> 1.66.
+constexpr int kTensorMaxShift = 3;
+constexpr double kTensorWaves = 8192.0;
+
 // Host-built tile list (used for the dense tensor, where tau = 0 and systems
 // are small).
 int prepare_host_tiles(rchem_ctx* ctx, double tau) {
@@ -1181,7 +1188,25 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
     qc.ntiles = static_cast<int>(ctx->tiles.size()) - qc.tile_begin;
     if (curX >= 0 && qc.ntiles > 0) ctx->hclasses.push_back(qc);
   };
-  for_each_task(ctx, tau, [&](int X, int Y, int i, int, int lo, int hi) {
+  // 1 << sh lanes to a quartet where a class's tiles are too few for the chip
+  std::vector<double> waves(kNumPairClasses * kNumPairClasses, 0.0);
+  std::vector<int> most(waves.size(), 0);
+  for_each_task(ctx, tau, [&](int X, int Y, int, int, int lo, int hi) {
+    waves[X * kNumPairClasses + Y] += (hi - lo + 63) / 64;
+  });
+  int rc = RCHEM_OK;
+  for (int X = 0; X < kNumPairClasses; ++X)
+    for (int Y = 0; Y < kNumPairClasses && rc == RCHEM_OK; ++Y) {
+      const int c = X * kNumPairClasses + Y;
+      if (waves[c] == 0.0) continue;
+      const QClass q = make_qclass(X, Y);
+      ClassKernel fn;
+      rc = class_kernel(ctx, q.la, q.lb, q.lc, q.ld, kModeTensor, kBoysExact, 0, &fn);
+      if (!fn.fn) continue;  // the other engines spread a quartet over a wave
+      while (most[c] < kTensorMaxShift && waves[c] * (2 << most[c]) <= kTensorWaves) ++most[c];
+    }
+  TRY(rc);
+  for_each_task(ctx, tau, [&](int X, int Y, int i, int b, int lo, int hi) {
     if (X != curX || Y != curY) {
       flush();
       curX = X;
@@ -1189,7 +1214,10 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
       qc = make_qclass(X, Y);
       qc.tile_begin = static_cast<int>(ctx->tiles.size());
     }
-    for (int j = lo; j < hi; j += 64) ctx->tiles.push_back(Tile{i, j, std::min(64, hi - j), 0});
+    int sh = most[X * kNumPairClasses + Y];
+    while (sh > 0 && (1 << sh) > ctx->buckets[Y][b].np) --sh;
+    const int w = 64 >> sh;
+    for (int j = lo; j < hi; j += w) ctx->tiles.push_back(Tile{i, j, std::min(w, hi - j), sh});
   });
   flush();
   for (const QClass& q : ctx->hclasses) {

@@ -1,0 +1,30 @@
+"""Tensor quartets on several lanes, nuclei over a pair's lanes, and the DIIS
+solve for small and large subspaces, against the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from rchem_amd import basis as rb
+from rchem_amd._lib import BOYS_EXACT, default_opts
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ls, npr", [
+    ([0], [1]),                         # one lane: one ket primitive pair
+    ([0, 0, 1], [1, 2, 3]),             # 1 .. 9 pairs: 1, 2, 4 and 8 lanes, remainders
+    ([0, 1, 1, 0, 0], [1, 1, 3, 7, 2]),  # 15, 10 and 21 kets: tiles of 8 and a few
+    ([2, 1, 0], [2, 1, 3]),             # d classes: per-lane and wave engines
+])
+def test_tensor_lanes_vs_oracle(gpu_ctx, ls, npr):
+    """Bar: 1e-11 of the largest integral, the parity bar of the d classes."""
+    rng = np.random.default_rng(len(ls))
+    ls, npr = np.array(ls, dtype=np.int32), np.array(npr, dtype=np.int32)
+    c = rng.uniform(-1.0, 1.0, (len(ls), 3))
+    ex = np.exp(rng.uniform(np.log(0.2), np.log(20.0), npr.sum()))
+    cf = rng.uniform(0.1, 1.0, npr.sum())
+    B = rb.Basis.from_shells(c, ls, npr, ex, cf, ctx=gpu_ctx)
+    print(f"case: l {ls.tolist()}, {npr.tolist()} primitives", flush=True)
+    I = rb.build_I(B, default_opts(boys_mode=BOYS_EXACT))
+    Io = O.eri_tensor(O.cgtos_from_shells(c, ls, npr, ex, cf), boys=O.BOYS_EXACT)
+    assert np.abs(I - Io).max() <= 1e-11 * max(1.0, np.abs(Io).max())
