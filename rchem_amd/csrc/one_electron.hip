@@ -1,7 +1,12 @@
 // One-electron integrals S, T, V over contracted Cartesian Gaussians (gfx950).
 //
-// One thread per shell pair (a >= b), one kernel per (la, lb) class, writes the
-// full component blocks of S, T and V and their transposes.  McMurchie--Davidson: per axis the Hermite
+// Eight lanes to a shell pair (a >= b), one kernel per (la, lb) class: each takes
+// every eighth nucleus (and all of S and T, a small share of the work), their
+// sums are added, and they write the full component blocks of S, T and V and
+// their transposes.  With one lane to a pair the kernels were bound by the chain
+// of primitive pairs x nuclei in a lane and by too few waves to cover it:
+// (H2O)_64 6-31G, (s|s) 1.53 -> 0.62 ms,
+// all classes 3.78 -> 1.10; (H2O)_8 (s|s) 0.20 -> 0.05.  McMurchie--Davidson: per axis the Hermite
 // expansion coefficients E_t^{ij}, overlap S_x(i,j) = E_0^{ij} sqrt(pi/p),
 // kinetic energy from overlaps with b shifted by +-2 (the identity rchem's
 // C library uses, cints.c:152-177), nuclear attraction
@@ -42,6 +47,8 @@ struct OneElArgs {
 };
 
 constexpr int kLmax1 = 2;              // highest l served
+constexpr int kOneElLanes = 8;         // lanes to a shell pair
+constexpr int kOneElBlock = 256;
 constexpr int kE = kLmax1 + 3;         // E index range for j up to lb + 2
 
 __device__ __forceinline__ int ncart1(int l) { return (l + 1) * (l + 2) / 2; }
@@ -138,15 +145,17 @@ __host__ __device__ constexpr int cart_z(int l, int k) {
 // coefficients and the R_tuv table live in registers; the Boys block of order
 // LA + LB is staged in LDS.
 template <int LA, int LB>
-__global__ __launch_bounds__(128) void one_electron_kernel(const OneElArgs a) {
+__global__ __launch_bounds__(kOneElBlock) void one_electron_kernel(const OneElArgs a) {
   constexpr int L = LA + LB;
   constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2;
   __shared__ __align__(16) double boys_tab[boys_stage_size(L)];
   stage_boys<L>(boys_tab, a.boys_table);
   __syncthreads();
   const int c = 3 * LA + LB;
-  const int pid = a.cls_begin[c] + static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-  if (pid >= a.cls_begin[c + 1]) return;
+  const int part = threadIdx.x % kOneElLanes;
+  const int pid = a.cls_begin[c] + static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) /
+                                                    kOneElLanes);
+  if (pid >= a.cls_begin[c + 1]) return;  // a pair's lanes together
   const int2 pr = a.pairs[pid];
   const ShellDev sa = a.shells[pr.x], sb = a.shells[pr.y];
   double s[NA][NB], t[NA][NB], v[NA][NB];
@@ -204,7 +213,7 @@ __global__ __launch_bounds__(128) void one_electron_kernel(const OneElArgs a) {
         }
       // nuclear attraction, one nucleus at a time: R_tuv by the Hermite recursion
       const double pre_v0 = -cc * kab * 2.0 * 3.14159265358979323846 * oop;
-      for (int cn = c0; cn < c1; ++cn) {
+      for (int cn = c0 + part; cn < c1; cn += kOneElLanes) {
         const double PC[3] = {P[0] - a.atom_xyz[3 * cn], P[1] - a.atom_xyz[3 * cn + 1],
                               P[2] - a.atom_xyz[3 * cn + 2]};
         const double T = p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
@@ -269,6 +278,10 @@ __global__ __launch_bounds__(128) void one_electron_kernel(const OneElArgs a) {
       int cb[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
       const double f = comp_factor(ca) * comp_factor(cb);
       const size_t mu = sa.f0 + i, nu = sb.f0 + j;
+#pragma unroll
+      for (int off = kOneElLanes / 2; off > 0; off >>= 1)
+        v[i][j] += __shfl_xor(v[i][j], off, kOneElLanes);
+      if ((i * NB + j) % kOneElLanes != part) continue;
       if (a.S) { a.S[mu * n + nu] = f * s[i][j]; a.S[nu * n + mu] = f * s[i][j]; }
       if (a.T) { a.T[mu * n + nu] = f * t[i][j]; a.T[nu * n + mu] = f * t[i][j]; }
       if (a.V) { a.V[mu * n + nu] = f * v[i][j]; a.V[nu * n + mu] = f * v[i][j]; }
@@ -563,7 +576,8 @@ hipError_t one_electron_class(const OneElArgs& a, hipStream_t s) {
   const int c = 3 * LA + LB;
   const int cnt = a.cls_begin[c + 1] - a.cls_begin[c];
   if (cnt <= 0) return hipSuccess;
-  hipLaunchKernelGGL((one_electron_kernel<LA, LB>), dim3((cnt + 127) / 128), dim3(128), 0, s, a);
+  hipLaunchKernelGGL((one_electron_kernel<LA, LB>), dim3((cnt * kOneElLanes + kOneElBlock - 1) / kOneElBlock),
+                     dim3(kOneElBlock), 0, s, a);
   return hipGetLastError();
 }
 

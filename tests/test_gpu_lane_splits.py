@@ -28,3 +28,21 @@ def test_tensor_lanes_vs_oracle(gpu_ctx, ls, npr):
     I = rb.build_I(B, default_opts(boys_mode=BOYS_EXACT))
     Io = O.eri_tensor(O.cgtos_from_shells(c, ls, npr, ex, cf), boys=O.BOYS_EXACT)
     assert np.abs(I - Io).max() <= 1e-11 * max(1.0, np.abs(Io).max())
+
+
+@pytest.mark.parametrize("nuclei", [0, 1, 7, 8, 9, 33])
+def test_nuclei_over_lanes_vs_oracle(gpu_ctx, nuclei):
+    """Bar: 1e-12 per nucleus of unit charge and a few of rounding in S and T."""
+    rng = np.random.default_rng(nuclei)
+    ls = np.array([0, 1, 2, 1, 0], dtype=np.int32)
+    npr = np.array([3, 2, 1, 3, 1], dtype=np.int32)
+    c = rng.uniform(-1.5, 1.5, (5, 3))
+    ex = np.exp(rng.uniform(np.log(0.2), np.log(20.0), npr.sum()))
+    cf = rng.uniform(0.1, 1.0, npr.sum())
+    xyz, Z = rng.uniform(-3.0, 3.0, (nuclei, 3)), rng.integers(1, 9, nuclei).astype(float)
+    B = rb.Basis.from_shells(c, ls, npr, ex, cf, ctx=gpu_ctx)
+    print(f"case: {nuclei} nuclei", flush=True)
+    got = rb.one_electron(B, xyz, Z)
+    ref = O.one_electron(O.cgtos_from_shells(c, ls, npr, ex, cf), Z, xyz)
+    for a, b in zip(got, ref):
+        assert np.abs(a - b).max() <= 1e-12 * (1 + Z.sum()) * max(1.0, np.abs(ref[0]).max())
