@@ -46,3 +46,15 @@ def test_nuclei_over_lanes_vs_oracle(gpu_ctx, nuclei):
     ref = O.one_electron(O.cgtos_from_shells(c, ls, npr, ex, cf), Z, xyz)
     for a, b in zip(got, ref):
         assert np.abs(a - b).max() <= 1e-12 * (1 + Z.sum()) * max(1.0, np.abs(ref[0]).max())
+
+
+@pytest.mark.parametrize("k", [1, 2, 5, 31, 32])
+def test_diis_subspaces(gpu_ctx, k):
+    """The energy does not depend on the subspace: 1e-9 hartree at a threshold of 1e-11."""
+    Z = np.array([8, 1, 1])
+    xyz = np.array([[0.0, -0.1432, 0.0], [1.638, 1.1365, 0.0], [-1.638, 1.1365, 0.0]])
+    B = rb.Basis.new(Z, xyz, "6-31G", ctx=gpu_ctx)
+    ref, _ = rb.scf(B, xyz, Z, nocc=5, thresh_e=1e-11, diis=8)
+    print(f"case: {k} vectors", flush=True)
+    res, _ = rb.scf(B, xyz, Z, nocc=5, thresh_e=1e-11, diis=k)
+    assert res.converged and abs(res.e_total - ref.e_total) <= 1e-9
