@@ -167,13 +167,14 @@ struct OneElArgs {
 // boundaries, the order one_electron_launch expects.
 void sort_pairs_by_class(const std::vector<ShellDev>& sh, std::vector<int2>* pr, int* cls_begin) {
   auto cls = [&](const int2& q) { return 3 * sh[q.x].l + sh[q.y].l; };
-  std::stable_sort(pr->begin(), pr->end(),
-                   [&](const int2& x, const int2& y) { return cls(x) < cls(y); });
-  size_t i = 0;
-  for (int c = 0; c < 10; ++c) {
-    while (i < pr->size() && cls((*pr)[i]) < c) ++i;
-    cls_begin[c] = static_cast<int>(i);
-  }
+  std::fill(cls_begin, cls_begin + 10, 0);
+  for (const int2& q : *pr) ++cls_begin[cls(q) + 1];
+  for (int c = 1; c < 10; ++c) cls_begin[c] += cls_begin[c - 1];
+  std::vector<int2> out(pr->size());
+  int next[10];
+  std::copy(cls_begin, cls_begin + 10, next);
+  for (const int2& q : *pr) out[next[cls(q)]++] = q;
+  pr->swap(out);
 }
 struct OneElGradArgs {
   const ShellDev* shells;
@@ -283,7 +284,45 @@ struct PairHost {
   int a, b;     // shell indices, l(a) >= l(b)
   int cls, np;
   double Q;
+  double kmax;  // max |K_ab| of its primitive pairs
 };
+
+// Stable sort by falling Q (finite, not negative: their bits order as they do),
+// a radix sort of the inverted bits, 11 at a time.
+void sort_by_bound(std::vector<PairHost>* v, size_t begin, size_t end) {
+  const size_t n = end - begin;
+  if (n < 512) {
+    std::stable_sort(v->begin() + begin, v->begin() + end,
+                     [](const PairHost& x, const PairHost& y) { return x.Q > y.Q; });
+    return;
+  }
+  struct Key {
+    unsigned long long bits;
+    unsigned at;
+  };
+  std::vector<Key> a(n), b(n);
+  for (size_t i = 0; i < n; ++i) {
+    const double q = (*v)[begin + i].Q + 0.0;  // -0 as 0
+    std::memcpy(&a[i].bits, &q, sizeof(q));
+    a[i].bits = ~a[i].bits;
+    a[i].at = static_cast<unsigned>(i);
+  }
+  for (int shift = 0; shift < 64; shift += 11) {
+    size_t count[2048] = {};
+    for (const Key& k : a) ++count[(k.bits >> shift) & 2047];
+    if (count[(a[0].bits >> shift) & 2047] == n) continue;
+    size_t sum = 0;
+    for (size_t& c : count) {
+      const size_t x = c;
+      c = sum;
+      sum += x;
+    }
+    for (const Key& k : a) b[count[(k.bits >> shift) & 2047]++] = k;
+    a.swap(b);
+  }
+  const std::vector<PairHost> from(v->begin() + begin, v->begin() + end);
+  for (size_t i = 0; i < n; ++i) (*v)[begin + i] = from[a[i].at];
+}
 
 }  // namespace
 
@@ -329,7 +368,8 @@ struct rchem_ctx {
   double pairs_tau = -1.0;
   std::vector<PairRec> pairs;
   std::vector<double> pairQ;                      // Schwarz bound, layout order
-  std::vector<std::pair<int, int>> pair_shells;   // (a, b), layout order
+  std::vector<std::pair<int, int>> pair_shells;
+  std::vector<double> pair_kmax;  // max |K_ab| of each pair's primitive pairs (layout order)   // (a, b), layout order
   size_t nprims = 0;
   std::vector<Bucket> buckets[kNumPairClasses];
   int class_begin[kNumPairClasses + 1] = {0};
@@ -673,6 +713,27 @@ int finish_basis(rchem_ctx* ctx) {
   return RCHEM_OK;
 }
 
+// K_ab of two primitives: the product of their coefficients, the Gaussian
+// product's factor and the integral's constant.
+double prim_kab(const rchem_ctx* ctx, int p, int q, double AB2) {
+  const double al = ctx->exps[p], be = ctx->exps[q], z = al + be;
+  return ctx->ccoef[p] * ctx->ccoef[q] * std::sqrt(2.0) * std::pow(M_PI, 1.25) / z *
+         std::exp(-al * be / z * AB2);
+}
+
+// The number of them that make_prims keeps.
+int count_prims(const rchem_ctx* ctx, int a, int b, double eps) {
+  const Shell& sa = ctx->shells[a];
+  const Shell& sb = ctx->shells[b];
+  double AB2 = 0.0;
+  for (int x = 0; x < 3; ++x) AB2 += (sa.xyz[x] - sb.xyz[x]) * (sa.xyz[x] - sb.xyz[x]);
+  int n = 0;
+  for (int ip = 0; ip < sa.nprim; ++ip)
+    for (int jp = 0; jp < sb.nprim; ++jp)
+      n += !(std::fabs(prim_kab(ctx, sa.p0 + ip, sb.p0 + jp, AB2)) < eps);
+  return n;
+}
+
 // Primitive pairs of shell pair (a, b) whose |K_ab| reaches eps (all of them
 // when eps <= 0), in (i of a, j of b) order.
 void make_prims(const rchem_ctx* ctx, int a, int b, double eps, std::vector<PrimRec>* out,
@@ -693,8 +754,7 @@ void make_prims(const rchem_ctx* ctx, int a, int b, double eps, std::vector<Prim
       pr.pax = -be / z * (sa.xyz[0] - sb.xyz[0]);
       pr.pay = -be / z * (sa.xyz[1] - sb.xyz[1]);
       pr.paz = -be / z * (sa.xyz[2] - sb.xyz[2]);
-      pr.kab = ctx->ccoef[sa.p0 + ip] * ctx->ccoef[sb.p0 + jp] * std::sqrt(2.0) *
-               std::pow(M_PI, 1.25) / z * std::exp(-al * be / z * AB2);
+      pr.kab = prim_kab(ctx, sa.p0 + ip, sb.p0 + jp, AB2);
       pr.oo2z = 0.5 / z;
       if (eps > 0.0 && std::fabs(pr.kab) < eps) continue;
       out->push_back(pr);
@@ -708,29 +768,51 @@ void make_prims(const rchem_ctx* ctx, int a, int b, double eps, std::vector<Prim
 // Primitive pairs with |K_ab| < prim_eps are dropped (prim_eps <= 0 keeps all);
 // a pair left with none is dropped.
 int layout_pairs(rchem_ctx* ctx, const std::vector<PairHost>& sel, double prim_eps) {
-  std::vector<PairHost> v;
-  v.reserve(sel.size());
+  std::vector<PairHost> kept;
+  kept.reserve(sel.size());
   std::vector<PrimRec> tmp;
   for (const PairHost& p : sel) {
-    make_prims(ctx, p.a, p.b, prim_eps, &tmp);
-    if (tmp.empty()) continue;
     PairHost q = p;
-    q.np = static_cast<int>(tmp.size());
-    v.push_back(q);
+    q.np = prim_eps > 0.0 ? count_prims(ctx, p.a, p.b, prim_eps)
+                          : ctx->shells[p.a].nprim * ctx->shells[p.b].nprim;
+    if (q.np > 0) kept.push_back(q);
   }
   const bool multi = !ctx->shell_mol.empty();
   auto mol_of = [&](const PairHost& p) { return multi ? ctx->shell_mol[p.a] : 0; };
-  std::stable_sort(v.begin(), v.end(), [&](const PairHost& x, const PairHost& y) {
-    if (x.cls != y.cls) return x.cls < y.cls;
-    if (x.np != y.np) return x.np > y.np;
-    if (mol_of(x) != mol_of(y)) return mol_of(x) < mol_of(y);
-    return x.Q > y.Q;
-  });
+  // by class and falling primitive count in one counting sort, each bucket then
+  // by its bounds; the primitive pairs are evaluated three times over both layouts
+  // of a basis, not five: a first build of (H2O)_64 85 -> 72 ms, 48 molecules'
+  // SCF 75 -> 67 (kept from one layout to the next, they cost it 73)
+  int npmax = 0;
+  for (const PairHost& p : kept) npmax = std::max(npmax, p.np);
+  std::vector<size_t> place(static_cast<size_t>(kNumPairClasses) * (npmax + 1) + 1, 0);
+  auto bucket_of = [&](const PairHost& p) {
+    return static_cast<size_t>(p.cls) * (npmax + 1) + (npmax - p.np);
+  };
+  for (const PairHost& p : kept) ++place[bucket_of(p) + 1];
+  for (size_t b = 1; b < place.size(); ++b) place[b] += place[b - 1];
+  std::vector<PairHost> v(kept.size());
+  {
+    std::vector<size_t> next(place);
+    for (const PairHost& p : kept) v[next[bucket_of(p)]++] = p;
+  }
+  for (size_t b = 0; b + 1 < place.size(); ++b) {
+    if (place[b + 1] - place[b] < 2) continue;
+    if (multi)
+      std::stable_sort(v.begin() + place[b], v.begin() + place[b + 1],
+                       [&](const PairHost& x, const PairHost& y) {
+                         if (mol_of(x) != mol_of(y)) return mol_of(x) < mol_of(y);
+                         return x.Q > y.Q;
+                       });
+    else
+      sort_by_bound(&v, place[b], place[b + 1]);
+  }
   ctx->pair_mol.resize(v.size());
   for (size_t k = 0; k < v.size(); ++k) ctx->pair_mol[k] = mol_of(v[k]);
   ctx->pairs.assign(v.size(), PairRec{});
   ctx->pairQ.resize(v.size());
   ctx->pair_shells.resize(v.size());
+  ctx->pair_kmax.assign(v.size(), 0.0);
   std::vector<PrimRec> prims;
   std::vector<double> alphas, tmp_alpha;
   for (int c = 0; c < kNumPairClasses; ++c) ctx->buckets[c].clear();
@@ -768,6 +850,7 @@ int layout_pairs(rchem_ctx* ctx, const std::vector<PairHost>& sel, double prim_e
       make_prims(ctx, ph.a, ph.b, prim_eps, &tmp, &tmp_alpha);
       for (int k = 0; k < np; ++k) {
         prims[base + static_cast<size_t>(k) * n + q] = tmp[k];
+        ctx->pair_kmax[pos + q] = std::max(ctx->pair_kmax[pos + q], std::fabs(tmp[k].kab));
         alphas[base + static_cast<size_t>(k) * n + q] = tmp_alpha[k];
       }
     }
@@ -1019,7 +1102,7 @@ int compute_schwarz(rchem_ctx* ctx) {
       int x = a, y = b;
       if (ctx->shells[y].l > ctx->shells[x].l) std::swap(x, y);
       all.push_back(PairHost{x, y, pair_class(ctx->shells[x].l, ctx->shells[y].l),
-                             ctx->shells[x].nprim * ctx->shells[y].nprim, 0.0});
+                             ctx->shells[x].nprim * ctx->shells[y].nprim, 0.0, 0.0});
     }
   TRY(layout_pairs(ctx, all, 0.0));
   // diagonal tiles: 64 consecutive pairs of one bucket, bra = ket per lane
@@ -1068,7 +1151,7 @@ int compute_schwarz(rchem_ctx* ctx) {
       return ctx->fail(RCHEM_ERR_NONFINITE, "non-finite Schwarz bound");
     const int a = ctx->pair_shells[i].first, b = ctx->pair_shells[i].second;
     sorted[i] = PairHost{a, b, pair_class(ctx->shells[a].l, ctx->shells[b].l),
-                         ctx->shells[a].nprim * ctx->shells[b].nprim, Q[i]};
+                         ctx->shells[a].nprim * ctx->shells[b].nprim, Q[i], ctx->pair_kmax[i]};
   }
   ctx->all_pairs = std::move(sorted);
   ctx->have_schwarz = true;
@@ -1103,13 +1186,8 @@ int prepare_pairs(rchem_ctx* ctx, double tau) {
   // times factors of order one; dropping |K_ab| < 1e-3 tau / K_max keeps every
   // dropped primitive quartet three orders below the quartet threshold.
   double kmax = 0.0;
-  if (tau > 0.0) {
-    std::vector<PrimRec> tmp;
-    for (const auto& p : sel) {
-      make_prims(ctx, p.a, p.b, 0.0, &tmp);
-      for (const auto& pr : tmp) kmax = std::max(kmax, std::fabs(pr.kab));
-    }
-  }
+  if (tau > 0.0)
+    for (const auto& p : sel) kmax = std::max(kmax, p.kmax);
   const double prim_eps = (tau > 0.0 && kmax > 0.0) ? 1e-3 * tau / kmax : 0.0;
   TRY(layout_pairs(ctx, sel, prim_eps));
   ctx->pairs_tau = tau;
@@ -2568,6 +2646,7 @@ int rchem_one_electron(rchem_ctx* ctx, int natom, const double* Z, const double*
     sh[s].f0 = ctx->shells[s].f0;
   }
   std::vector<int2> pr;
+  pr.reserve(static_cast<size_t>(ns) * (ns + 1) / 2);
   for (int a = 0; a < ns; ++a)
     for (int b = 0; b <= a; ++b) pr.push_back(make_int2(a, b));
   int cls_begin[10];
