@@ -124,9 +124,9 @@ __device__ __forceinline__ void eri_compute(const TileSrc& src, const Tile t, co
   constexpr int L = C::L;
   constexpr bool KP = MODE == kModeJK;
   static_assert(BM == kBoysExact || sizeof(R) == 8, "compat Boys is FP64 only");
-  // kModeTensor: 1 << sh lanes to a quartet, each with every (1 << sh)-th ket
-  // primitive pair
-  constexpr bool SPLIT = MODE == kModeTensor;
+  // kModeTensor, kModeDiag: 1 << sh lanes to a quartet, each with every
+  // (1 << sh)-th ket primitive pair
+  constexpr bool SPLIT = MODE == kModeTensor || MODE == kModeDiag;
   const int sh = SPLIT ? t.pad : 0;
   const int part = SPLIT ? lane & ((1 << sh) - 1) : 0;
   const int q = SPLIT ? lane >> sh : lane;

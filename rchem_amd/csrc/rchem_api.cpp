@@ -1089,6 +1089,14 @@ void class_ls(int X, int* l1, int* l2) {
       }
 }
 
+// Lanes to a quartet of the tensor and Schwarz kernels: at most 8, and no more
+// than give the class (a bucket of it) 8 waves to a SIMD.  A lane's chain of
+// primitive quartets was the time of a small tensor's kernels: (H2O)_3 6-31G
+// (ss|ss) 0.289 -> 0.080 ms, all classes 0.89 -> 0.23, the call 2.35 -> 1.66; of
+// the bounds of (H2O)_8, (ss|ss) and (ps|ps): 0.42 and 0.14 -> 0.07 and 0.03 ms.
+constexpr int kTensorMaxShift = 3;
+constexpr double kTensorWaves = 8192.0;
+
 // Schwarz bounds for every shell pair (exact Boys), once per basis.
 int compute_schwarz(rchem_ctx* ctx) {
   if (ctx->have_schwarz) return RCHEM_OK;
@@ -1105,14 +1113,24 @@ int compute_schwarz(rchem_ctx* ctx) {
                              ctx->shells[x].nprim * ctx->shells[y].nprim, 0.0, 0.0});
     }
   TRY(layout_pairs(ctx, all, 0.0));
-  // diagonal tiles: 64 consecutive pairs of one bucket, bra = ket per lane
+  // diagonal tiles: up to 64 consecutive pairs of one bucket, bra = ket per lane
   ctx->tiles.clear();
   std::vector<std::pair<int, int>> ranges;  // per class: tile range
   for (int X = 0; X < kNumPairClasses; ++X) {
     const int t0 = static_cast<int>(ctx->tiles.size());
-    for (const Bucket& bk : ctx->buckets[X])
-      for (int j = bk.begin; j < bk.end; j += 64)
-        ctx->tiles.push_back(Tile{-1, j, std::min(64, bk.end - j), 0});
+    int l1, l2;
+    class_ls(X, &l1, &l2);
+    ClassKernel k;
+    TRY(class_kernel(ctx, l1, l2, l1, l2, kModeDiag, kBoysExact, 0, &k));
+    for (const Bucket& bk : ctx->buckets[X]) {
+      int sh = 0;
+      while (k.fn && sh < kTensorMaxShift && (2 << sh) <= bk.np &&
+             (bk.end - bk.begin) / 64.0 * (2 << sh) <= kTensorWaves)
+        ++sh;
+      const int w = 64 >> sh;
+      for (int j = bk.begin; j < bk.end; j += w)
+        ctx->tiles.push_back(Tile{-1, j, std::min(w, bk.end - j), sh});
+    }
     ranges.emplace_back(t0, static_cast<int>(ctx->tiles.size()) - t0);
   }
   TRY(upload_tiles(ctx));
@@ -1245,13 +1263,6 @@ double per_prim_flops(const QClass& qc, int* hrr) {
   *hrr = fh;
   return fv + 68.0 + 4.0 * (qc.la + qc.lb + qc.lc + qc.ld);
 }
-
-// Lanes to a quartet of the tensor kernels: at most 8, and no more than give the
-// class 8 waves to a SIMD.  A lane's chain of
-// primitive quartets was the time of a small tensor's kernels: (H2O)_3 6-31G
-// (ss|ss) 0.289 -> 0.080 ms, all classes 0.89 -> 0.23, the call 2.35 -> 1.66.
-constexpr int kTensorMaxShift = 3;
-constexpr double kTensorWaves = 8192.0;
 
 // Host-built tile list (used for the dense tensor, where tau = 0 and systems
 // are small).

@@ -30,6 +30,32 @@ def test_tensor_lanes_vs_oracle(gpu_ctx, ls, npr):
     assert np.abs(I - Io).max() <= 1e-11 * max(1.0, np.abs(Io).max())
 
 
+@pytest.mark.parametrize("ls, npr", [
+    ([0], [1]),
+    ([0, 0, 1], [1, 2, 7]),              # 1 .. 49 pairs of primitives
+    ([2, 1, 0, 0, 0, 0], [2, 1, 3, 3, 3, 3]),  # 10 (ss| pairs of one bucket: a tile and a few
+])
+def test_schwarz_lanes_vs_oracle(gpu_ctx, ls, npr):
+    """Bar: 1e-11 of the largest integral on the squares of the bounds."""
+    rng = np.random.default_rng(len(ls))
+    ls, npr = np.array(ls, dtype=np.int32), np.array(npr, dtype=np.int32)
+    c = rng.uniform(-1.0, 1.0, (len(ls), 3))
+    ex = np.exp(rng.uniform(np.log(0.2), np.log(20.0), npr.sum()))
+    cf = rng.uniform(0.1, 1.0, npr.sum())
+    B = rb.Basis.from_shells(c, ls, npr, ex, cf, ctx=gpu_ctx)
+    print(f"case: l {ls.tolist()}, {npr.tolist()} primitives", flush=True)
+    Q = rb.schwarz(B)
+    n = B.nbf
+    I = np.asarray(O.eri_tensor(O.cgtos_from_shells(c, ls, npr, ex, cf),
+                                boys=O.BOYS_EXACT)).reshape(n, n, n, n)
+    d = np.abs(np.einsum("ijij->ij", I))
+    f = np.concatenate([[0], np.cumsum((ls + 1) * (ls + 2) // 2)])
+    for a in range(len(ls)):
+        for b in range(a + 1):  # the lower triangle
+            ref = d[f[a]:f[a + 1], f[b]:f[b + 1]].max()
+            assert abs(Q[a, b] ** 2 - ref) <= 1e-11 * max(1.0, np.abs(I).max())
+
+
 @pytest.mark.parametrize("nuclei", [0, 1, 7, 8, 9, 33])
 def test_nuclei_over_lanes_vs_oracle(gpu_ctx, nuclei):
     """Bar: 1e-12 per nucleus of unit charge and a few of rounding in S and T."""
