@@ -634,7 +634,7 @@ def main():
         scf["note"] = ("DIIS(8); mixed switches to all-FP64 J/K once |dE| < 1e-7 Eh; "
                        "convergence |dE| < 1e-10 Eh and max|FDS-SDF| < 1e-8; 'seconds' "
                        "replays the captured Fock build (hipGraph) on every iteration and "
-                       "forms each iteration's density by canonical purification (DGEMM) "
+                       "forms each iteration's density by trace-correcting purification "
                        "instead of the eigensolver")
         out["scf"] = scf
     if not args.no_cpu_baseline and args.workload == "h2o64":

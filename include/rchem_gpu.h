@@ -251,7 +251,7 @@ typedef struct rchem_scf_opts {
                           kernel by kernel */
   int purify;          /* 1: each iteration's density D = X P X^T with P, the projector
                           onto the nocc lowest eigenvectors of F' = X^T F X, from
-                          canonical purification (GEMMs only) instead of the
+                          purification (products only) instead of the
                           eigensolver, which takes over only an iteration whose F'
                           has no gap.  Single-molecule SCF and gradient (whose
                           energy-weighted density is W = D F D either way); the

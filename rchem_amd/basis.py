@@ -206,7 +206,7 @@ def scf(basis: Basis, atomcoords, atomnos, nocc, thresh_e=1e-11, max_iter=1024,
     """rchem.rs:10-90 on the device: returns (SCFResult, D).  diis = k > 0
     replaces rchem's plain iterations by DIIS over k Fock matrices; graph
     replays the Fock build as a hipGraph; purify forms each iteration's
-    density by canonical purification (GEMMs) instead of the eigensolver."""
+    density by purification (products) instead of the eigensolver."""
     o = SCFOpts()
     lib().rchem_scf_opts_default(ctypes.byref(o))
     o.diis = int(diis)

@@ -19,12 +19,14 @@
 // streaming kernel (eri_stream.hpp: one wave to a quartet, lanes on its
 // primitives, every target summed over the wave through LDS, the recurrence and
 // the digestion of one quartet at a time by tables) waited for LDS with one wave
-// on a SIMD: VALU 0.22-0.31 of the cycles; here 0.62-0.71, which is the bound,
+// on a SIMD: VALU 0.22-0.31 of the cycles; here 0.64-0.75 (0.52 in
+// (dd|dd), one wave on a SIMD), which is the bound,
 // with the product and Boys work that each part repeats (130 of 535 vector
 // instructions of a (dp|dp) part) the larger part of the excess.  A build of 210
 // s/p/d shells of 3 primitives (n = 430), ms, per-lane or streaming and now:
 // (dp|pp) 17.6, 15.5; (dp|dp) 68.6, 16.2; (dd|ds) 20.5, 8.9; (dd|pp) 42.0, 8.6;
-// (dd|dp) 55.0, 18.1; (dd|dd) 32.0, 6.9.  The build: 267 -> 133.
+// (dd|dp) 55.0, 18.1; (dd|dd) 32.0, 6.9.  The build: 271 -> 133, and 127 with the
+// chunks handed out by a counter.
 // The recurrences are chgp.c:412-586 (VRR) and chgp.c:44-135 (HRR).
 #pragma once
 #include "eri_common.hpp"

@@ -1,5 +1,7 @@
 // Streaming ERI kernel for the classes whose contracted accumulators do not fit
-// one lane (total angular momentum L >= 5: (dp|pp) ... (dd|dd)).
+// one lane (total angular momentum L >= 5: (dp|pp) ... (dd|dd)): their bounds,
+// tensors and single quartets, and their Fock builds where the partwise kernel
+// (eri_part.hpp) is switched off.
 //
 // One wavefront evaluates one contracted shell quartet at a time, one
 // primitive quartet per lane (64 at a time; a quartet with more runs in

@@ -19,6 +19,7 @@
 //              radix-sorted by first ket pair within each class); per class the
 //              [begin, end) tile and chunk ranges of each precision go to device
 //              memory, where the persistent ERI kernels read them.
+// Small passes take 2 to 5 in one launch (plan_direct_kernel).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 

@@ -142,7 +142,7 @@ __host__ __device__ constexpr int cart_z(int l, int k) {
   return 0;
 }
 
-// One thread per shell pair of class (LA, LB): pairs [cls_begin[c], cls_begin[c + 1]),
+// kOneElLanes lanes to a shell pair of class (LA, LB): pairs [cls_begin[c], cls_begin[c + 1]),
 // c = 3 LA + LB.  Every loop has compile-time bounds, so the Hermite
 // coefficients and the R_tuv table live in registers; the Boys block of order
 // LA + LB is staged in LDS.

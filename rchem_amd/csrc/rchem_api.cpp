@@ -1024,7 +1024,8 @@ int find_program(rchem_ctx* ctx, int la, int lb, int lc, int ld, int grad,
 // wave-cooperative): (dp|dp) 138 vs 246, (dd|pp) 78 vs 150, (dd|dp) 84 vs 470,
 // (dd|dd) 37 vs 113; the per-lane kernels keep (dp|pp) 125 vs 174, (dp|ds) 52
 // vs 142, (dd|ps) 17 vs 72, (dd|ds) 53 vs 62.  RCHEM_ERI_STREAM=0: never, 2:
-// every class it serves (also in place of LDS digestion).
+// every class it serves (also in place of LDS digestion); either switches off
+// the partwise Fock-build kernels, which are faster than both (eri_part.hpp).
 bool stream_preferred(const rchem_ctx* ctx, int la, int lb, int lc, int ld) {
   const int key = ((la * 10 + lb) * 10 + lc) * 10 + ld;
   return ctx->eri_stream_mode == 2 ||
@@ -1339,8 +1340,6 @@ int split_limit(const QClass& qc, double iters) {
 // tiles / 1024 (at least 8): (H2O)_8 1.06 -> 0.84 ms, water 0.26 -> 0.19.
 constexpr double kMinChunks = 1024.0;
 
-// Device-planner tables for threshold tau: classes, buckets, capacities and
-// the FP64 statistics (exact for all-FP64 builds).
 // Passes of at most this many tiles are planned in one launch, a class's units
 // in any order.  The scans and sorts of the ordered plan are some ten launches
 // (FP64 water STO-3G 0.185 -> 0.155 ms, its 27-iteration SCF 7.2 -> 6.5 ms), but
@@ -1351,6 +1350,8 @@ constexpr double kMinChunks = 1024.0;
 constexpr int kDirectPlanTiles = 65536;
 constexpr double kPassTiles = 67108864.0;  // 2^26 tiles (1 GiB per tile list) per pass
 
+// Device-planner tables for threshold tau: classes, buckets, capacities and
+// the FP64 statistics (exact for all-FP64 builds).
 int prepare_plan(rchem_ctx* ctx, double tau) {
   TRY(prepare_pairs(ctx, tau));
   if (ctx->plan_tau == tau) return RCHEM_OK;
