@@ -14,6 +14,7 @@ using EriLaunchFn = hipError_t (*)(const EriArgs&, int, hipStream_t);
 struct EriPart {
   hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
   size_t (*slab)(int cus) = nullptr;
+  bool (*rows_fit)(int kw) = nullptr;
 };
 
 #include "generated/eri_dispatch.inc"

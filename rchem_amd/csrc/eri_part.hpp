@@ -332,14 +332,26 @@ hipError_t eri_part_launch_rows(const EriArgs& a, double* slab, size_t lds, int 
   return hipGetLastError();
 }
 
+// LDS of a workgroup beside its rows, and whether its K rows of kw columns fit.
+template <int LA, int LB, int LC, int LD>
+constexpr size_t eri_part_fixed() {
+  return sizeof(double) * (part_boys<LA + LB + LC + LD>() + ncart(LC) * ncart(LD) * 64 +
+                           ncart(LA) * ncart(LB));
+}
+template <int LA, int LB, int LC, int LD>
+bool eri_part_rows_fit(int kw) {
+  return eri_part_fixed<LA, LB, LC, LD>() +
+             sizeof(double) * (ncart(LA) + ncart(LB)) * static_cast<size_t>(kw) <=
+         kLdsPerCu;
+}
+
 template <int LA, int LB, int LC, int LD>
 hipError_t eri_part_launch(const EriArgs& a, double* slab, size_t bytes, int cus, hipStream_t s) {
-  constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+  constexpr int NA = ncart(LA), NB = ncart(LB);
   constexpr int groups = part_groups<LA, LB, LC, LD>();
   if (!a.Dp || !a.Jp || !slab || eri_part_slab<LA, LB, LC, LD>(cus) > bytes)
     return hipErrorInvalidValue;
-  const size_t fixed =
-      sizeof(double) * (part_boys<LA + LB + LC + LD>() + NC * ND * 64 + NA * NB);
+  const size_t fixed = eri_part_fixed<LA, LB, LC, LD>();
   const size_t rows = sizeof(double) * (NA + NB) * static_cast<size_t>(a.kw);
   // K rows in LDS where they fit, the density's too unless that costs a workgroup
   const auto held = [&](size_t lds) { return std::min<int>(groups, kLdsPerCu / lds); };

@@ -44,10 +44,12 @@ hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s);
 EriLaunchFn eri_jk_lds_launcher(int la, int lb, int lc, int ld, int bm, int fp32, int v);
 EriStreamFn eri_stream_launcher(int la, int lb, int lc, int ld, int mode);
 // Partwise Fock-build kernel of a class: its launcher and the bytes of global
-// memory its workgroups keep a tile's accumulators in.
+// memory its workgroups keep a tile's accumulators in, and whether the K rows of
+// kw columns fit the LDS.
 struct EriPart {
   hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
   size_t (*slab)(int cus) = nullptr;
+  bool (*rows_fit)(int kw) = nullptr;
 };
 EriPart eri_part_launcher(int la, int lb, int lc, int ld);
 hipError_t eri_generic_launch(const EriArgs& a, const GenericProgram& p, int mode, int bm,
@@ -1042,9 +1044,15 @@ int class_kernel(rchem_ctx* ctx, int la, int lb, int lc, int ld, int mode, int b
   if (!ctx->force_generic) {
     const bool prefer = stream_preferred(ctx, la, lb, lc, ld);
     // a Fock build's FP64 quartets of L >= 5, and the FP32 list of the classes
-    // without an FP32 kernel of their own
+    // without an FP32 kernel of their own.  (dp|pp) and (dd|ds) only while their K
+    // rows are in LDS: with K in memory they took 47.5 and 28.0 ms (210 shells,
+    // n = 430) where the per-lane kernels take 17.6 and 20.5, while the classes
+    // that otherwise stream gain either way ((dp|dp) 33.5 against 68.6)
     if (ctx->eri_stream_mode == 1 && mode == kModeJK && bm == kBoysExact && (!fp32 || prefer)) {
       out->part = eri_part_launcher(la, lb, lc, ld);
+      const int kw = ctx->shell_mol.empty() ? ctx->nbf : ctx->mol_kw;
+      if (out->part.launch && !prefer && !(ctx->lds_digestion && out->part.rows_fit(kw)))
+        out->part = EriPart{};
       if (out->part.launch) {
         out->slab = ctx->part_slab_d.as<double>();
         out->slab_bytes = ctx->part_slab_d.bytes;
