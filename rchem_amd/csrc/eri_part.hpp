@@ -145,6 +145,7 @@ __global__ __launch_bounds__(THREADS, MINW) void eri_part_kernel(
   for (int k = tid; k < NC * ND * 64; k += THREADS) jq[k] = 0.0;
   const int begin = ROWS ? a.chunk_range[0] : a.tile_range ? a.tile_range[0] : 0;
   const int end = ROWS ? a.chunk_range[1] : a.tile_range ? a.tile_range[1] : a.ntiles;
+  __syncthreads();  // the staged table is complete before a wave's first lookup
   __shared__ int s_next[2];  // by turns: a chunk may have no barrier but its last
   int turn = 0;
   for (int u = begin + static_cast<int>(blockIdx.x); u < end;) {  // block-uniform
