@@ -21,6 +21,7 @@
 #include <algorithm>
 
 #include "boys.hpp"
+#include "one_electron_launch.hpp"
 
 namespace rchem {
 
@@ -49,8 +50,6 @@ struct OneElArgs {
 };
 
 constexpr int kLmax1 = 2;              // highest l served
-constexpr int kOneElLanes = 8;         // lanes to a shell pair
-constexpr int kOneElBlock = 256;
 constexpr int kE = kLmax1 + 3;         // E index range for j up to lb + 2
 
 __device__ __forceinline__ int ncart1(int l) { return (l + 1) * (l + 2) / 2; }
@@ -155,139 +154,141 @@ __global__ __launch_bounds__(kOneElBlock) void one_electron_kernel(const OneElAr
   __syncthreads();
   const int c = 3 * LA + LB;
   const int part = threadIdx.x % kOneElLanes;
-  const int pid = a.cls_begin[c] + static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) /
-                                                    kOneElLanes);
-  if (pid >= a.cls_begin[c + 1]) return;  // a pair's lanes together
-  const int2 pr = a.pairs[pid];
-  const ShellDev sa = a.shells[pr.x], sb = a.shells[pr.y];
-  double s[NA][NB], t[NA][NB], v[NA][NB];
+  const long long count = a.cls_begin[c + 1] - a.cls_begin[c];
+  // a pair's lanes leave together
+  for (long long p = one_el_first(blockIdx.x, threadIdx.x); p < count; p += one_el_step(gridDim.x)) {
+    const int pid = a.cls_begin[c] + static_cast<int>(p);
+    const int2 pr = a.pairs[pid];
+    const ShellDev sa = a.shells[pr.x], sb = a.shells[pr.y];
+    double s[NA][NB], t[NA][NB], v[NA][NB];
 #pragma unroll
-  for (int i = 0; i < NA; ++i)
+    for (int i = 0; i < NA; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) s[i][j] = t[i][j] = v[i][j] = 0.0;
-  const double AB2 = (sa.xyz[0] - sb.xyz[0]) * (sa.xyz[0] - sb.xyz[0]) +
-                     (sa.xyz[1] - sb.xyz[1]) * (sa.xyz[1] - sb.xyz[1]) +
-                     (sa.xyz[2] - sb.xyz[2]) * (sa.xyz[2] - sb.xyz[2]);
-  int c0 = 0, c1 = a.natom;
-  if (a.shell_mol) {  // the pair's own molecule's nuclei
-    const int2 r = a.mol_atoms[a.shell_mol[pr.x]];
-    c0 = r.x;
-    c1 = r.y;
-  }
-  double E[3][LA + 1][LB + 3][L + 3];
-  for (int ip = 0; ip < sa.nprim; ++ip)
-    for (int jp = 0; jp < sb.nprim; ++jp) {
-      const double al = a.exps[sa.p0 + ip], be = a.exps[sb.p0 + jp];
-      const double p = al + be, oop = 1.0 / p;
-      const double cc = a.ccoef[sa.p0 + ip] * a.ccoef[sb.p0 + jp];
-      const double kab = exp(-al * be * oop * AB2);
-      double P[3];
+      for (int j = 0; j < NB; ++j) s[i][j] = t[i][j] = v[i][j] = 0.0;
+    const double AB2 = (sa.xyz[0] - sb.xyz[0]) * (sa.xyz[0] - sb.xyz[0]) +
+                       (sa.xyz[1] - sb.xyz[1]) * (sa.xyz[1] - sb.xyz[1]) +
+                       (sa.xyz[2] - sb.xyz[2]) * (sa.xyz[2] - sb.xyz[2]);
+    int c0 = 0, c1 = a.natom;
+    if (a.shell_mol) {  // the pair's own molecule's nuclei
+      const int2 r = a.mol_atoms[a.shell_mol[pr.x]];
+      c0 = r.x;
+      c1 = r.y;
+    }
+    double E[3][LA + 1][LB + 3][L + 3];
+    for (int ip = 0; ip < sa.nprim; ++ip)
+      for (int jp = 0; jp < sb.nprim; ++jp) {
+        const double al = a.exps[sa.p0 + ip], be = a.exps[sb.p0 + jp];
+        const double p = al + be, oop = 1.0 / p;
+        const double cc = a.ccoef[sa.p0 + ip] * a.ccoef[sb.p0 + jp];
+        const double kab = exp(-al * be * oop * AB2);
+        double P[3];
 #pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        P[x] = (al * sa.xyz[x] + be * sb.xyz[x]) * oop;
-        hermite_e_t<LA, LB + 2>(P[x] - sa.xyz[x], P[x] - sb.xyz[x], 0.5 * oop, E[x]);
-      }
-      const double sq = sqrt(3.14159265358979323846 * oop);
-      const double pre_s = cc * kab * sq * sq * sq;
-      // overlap and kinetic (b shifted by +-2, cints.c:152-177)
-#pragma unroll
-      for (int i = 0; i < NA; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          const int A[3] = {cart_x(LA, i), cart_y(LA, i), cart_z(LA, i)};
-          const int B[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
-          double ov[3], ovp2[3], ovm2[3];
-#pragma unroll
-          for (int x = 0; x < 3; ++x) {
-            ov[x] = E[x][A[x]][B[x]][0];
-            ovp2[x] = E[x][A[x]][B[x] + 2][0];
-            ovm2[x] = B[x] >= 2 ? E[x][A[x]][B[x] >= 2 ? B[x] - 2 : 0][0] : 0.0;
-          }
-          const double s0 = ov[0] * ov[1] * ov[2];
-          s[i][j] += pre_s * s0;
-          const int lbt = B[0] + B[1] + B[2];
-          const double t1 =
-              ovp2[0] * ov[1] * ov[2] + ov[0] * ovp2[1] * ov[2] + ov[0] * ov[1] * ovp2[2];
-          const double t2 = B[0] * (B[0] - 1) * ovm2[0] * ov[1] * ov[2] +
-                            B[1] * (B[1] - 1) * ov[0] * ovm2[1] * ov[2] +
-                            B[2] * (B[2] - 1) * ov[0] * ov[1] * ovm2[2];
-          t[i][j] += pre_s * (be * (2 * lbt + 3) * s0 - 2.0 * be * be * t1 - 0.5 * t2);
+        for (int x = 0; x < 3; ++x) {
+          P[x] = (al * sa.xyz[x] + be * sb.xyz[x]) * oop;
+          hermite_e_t<LA, LB + 2>(P[x] - sa.xyz[x], P[x] - sb.xyz[x], 0.5 * oop, E[x]);
         }
-      // nuclear attraction, one nucleus at a time: R_tuv by the Hermite recursion
-      const double pre_v0 = -cc * kab * 2.0 * 3.14159265358979323846 * oop;
-      for (int cn = c0 + part; cn < c1; cn += kOneElLanes) {
-        const double PC[3] = {P[0] - a.atom_xyz[3 * cn], P[1] - a.atom_xyz[3 * cn + 1],
-                              P[2] - a.atom_xyz[3 * cn + 2]};
-        const double T = p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
-        double F[L + 1];
-        boys_exact<L, double>(T, boys_tab, F);
-        double R[L + 1][L + 1][L + 1][L + 1];
-        double m2p = 1.0;
-#pragma unroll
-        for (int n = 0; n <= L; ++n) {
-          R[n][0][0][0] = m2p * F[n];
-          m2p *= -2.0 * p;
-        }
-#pragma unroll
-        for (int n = L - 1; n >= 0; --n) {
-#pragma unroll
-          for (int tt = 0; tt <= L - n; ++tt)
-#pragma unroll
-            for (int uu = 0; uu <= L - n - tt; ++uu)
-#pragma unroll
-              for (int vv = 0; vv <= L - n - tt - uu; ++vv) {
-                if (tt + uu + vv == 0) continue;
-                double r;
-                if (tt > 0) {
-                  r = PC[0] * R[n + 1][tt - 1][uu][vv];
-                  if (tt > 1) r += (tt - 1) * R[n + 1][tt > 1 ? tt - 2 : 0][uu][vv];
-                } else if (uu > 0) {
-                  r = PC[1] * R[n + 1][tt][uu - 1][vv];
-                  if (uu > 1) r += (uu - 1) * R[n + 1][tt][uu > 1 ? uu - 2 : 0][vv];
-                } else {
-                  r = PC[2] * R[n + 1][tt][uu][vv - 1];
-                  if (vv > 1) r += (vv - 1) * R[n + 1][tt][uu][vv > 1 ? vv - 2 : 0];
-                }
-                R[n][tt][uu][vv] = r;
-              }
-        }
-        const double pre_v = a.atom_z[cn] * pre_v0;
+        const double sq = sqrt(3.14159265358979323846 * oop);
+        const double pre_s = cc * kab * sq * sq * sq;
+        // overlap and kinetic (b shifted by +-2, cints.c:152-177)
 #pragma unroll
         for (int i = 0; i < NA; ++i)
 #pragma unroll
           for (int j = 0; j < NB; ++j) {
             const int A[3] = {cart_x(LA, i), cart_y(LA, i), cart_z(LA, i)};
             const int B[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
-            double sum = 0.0;
+            double ov[3], ovp2[3], ovm2[3];
 #pragma unroll
-            for (int tt = 0; tt <= A[0] + B[0]; ++tt)
-#pragma unroll
-              for (int uu = 0; uu <= A[1] + B[1]; ++uu)
-#pragma unroll
-                for (int vv = 0; vv <= A[2] + B[2]; ++vv)
-                  sum += E[0][A[0]][B[0]][tt] * E[1][A[1]][B[1]][uu] * E[2][A[2]][B[2]][vv] *
-                         R[0][tt][uu][vv];
-            v[i][j] += pre_v * sum;
+            for (int x = 0; x < 3; ++x) {
+              ov[x] = E[x][A[x]][B[x]][0];
+              ovp2[x] = E[x][A[x]][B[x] + 2][0];
+              ovm2[x] = B[x] >= 2 ? E[x][A[x]][B[x] >= 2 ? B[x] - 2 : 0][0] : 0.0;
+            }
+            const double s0 = ov[0] * ov[1] * ov[2];
+            s[i][j] += pre_s * s0;
+            const int lbt = B[0] + B[1] + B[2];
+            const double t1 =
+                ovp2[0] * ov[1] * ov[2] + ov[0] * ovp2[1] * ov[2] + ov[0] * ov[1] * ovp2[2];
+            const double t2 = B[0] * (B[0] - 1) * ovm2[0] * ov[1] * ov[2] +
+                              B[1] * (B[1] - 1) * ov[0] * ovm2[1] * ov[2] +
+                              B[2] * (B[2] - 1) * ov[0] * ov[1] * ovm2[2];
+            t[i][j] += pre_s * (be * (2 * lbt + 3) * s0 - 2.0 * be * be * t1 - 0.5 * t2);
           }
+        // nuclear attraction, one nucleus at a time: R_tuv by the Hermite recursion
+        const double pre_v0 = -cc * kab * 2.0 * 3.14159265358979323846 * oop;
+        for (int cn = c0 + part; cn < c1; cn += kOneElLanes) {
+          const double PC[3] = {P[0] - a.atom_xyz[3 * cn], P[1] - a.atom_xyz[3 * cn + 1],
+                                P[2] - a.atom_xyz[3 * cn + 2]};
+          const double T = p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]);
+          double F[L + 1];
+          boys_exact<L, double>(T, boys_tab, F);
+          double R[L + 1][L + 1][L + 1][L + 1];
+          double m2p = 1.0;
+#pragma unroll
+          for (int n = 0; n <= L; ++n) {
+            R[n][0][0][0] = m2p * F[n];
+            m2p *= -2.0 * p;
+          }
+#pragma unroll
+          for (int n = L - 1; n >= 0; --n) {
+#pragma unroll
+            for (int tt = 0; tt <= L - n; ++tt)
+#pragma unroll
+              for (int uu = 0; uu <= L - n - tt; ++uu)
+#pragma unroll
+                for (int vv = 0; vv <= L - n - tt - uu; ++vv) {
+                  if (tt + uu + vv == 0) continue;
+                  double r;
+                  if (tt > 0) {
+                    r = PC[0] * R[n + 1][tt - 1][uu][vv];
+                    if (tt > 1) r += (tt - 1) * R[n + 1][tt > 1 ? tt - 2 : 0][uu][vv];
+                  } else if (uu > 0) {
+                    r = PC[1] * R[n + 1][tt][uu - 1][vv];
+                    if (uu > 1) r += (uu - 1) * R[n + 1][tt][uu > 1 ? uu - 2 : 0][vv];
+                  } else {
+                    r = PC[2] * R[n + 1][tt][uu][vv - 1];
+                    if (vv > 1) r += (vv - 1) * R[n + 1][tt][uu][vv > 1 ? vv - 2 : 0];
+                  }
+                  R[n][tt][uu][vv] = r;
+                }
+          }
+          const double pre_v = a.atom_z[cn] * pre_v0;
+#pragma unroll
+          for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+              const int A[3] = {cart_x(LA, i), cart_y(LA, i), cart_z(LA, i)};
+              const int B[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
+              double sum = 0.0;
+#pragma unroll
+              for (int tt = 0; tt <= A[0] + B[0]; ++tt)
+#pragma unroll
+                for (int uu = 0; uu <= A[1] + B[1]; ++uu)
+#pragma unroll
+                  for (int vv = 0; vv <= A[2] + B[2]; ++vv)
+                    sum += E[0][A[0]][B[0]][tt] * E[1][A[1]][B[1]][uu] * E[2][A[2]][B[2]][vv] *
+                           R[0][tt][uu][vv];
+              v[i][j] += pre_v * sum;
+            }
+        }
       }
-    }
-  const size_t n = static_cast<size_t>(a.nbf);
+    const size_t n = static_cast<size_t>(a.nbf);
 #pragma unroll
-  for (int i = 0; i < NA; ++i)
+    for (int i = 0; i < NA; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      int ca[3] = {cart_x(LA, i), cart_y(LA, i), cart_z(LA, i)};
-      int cb[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
-      const double f = comp_factor(ca) * comp_factor(cb);
-      const size_t mu = sa.f0 + i, nu = sb.f0 + j;
+      for (int j = 0; j < NB; ++j) {
+        int ca[3] = {cart_x(LA, i), cart_y(LA, i), cart_z(LA, i)};
+        int cb[3] = {cart_x(LB, j), cart_y(LB, j), cart_z(LB, j)};
+        const double f = comp_factor(ca) * comp_factor(cb);
+        const size_t mu = sa.f0 + i, nu = sb.f0 + j;
 #pragma unroll
-      for (int off = kOneElLanes / 2; off > 0; off >>= 1)
-        v[i][j] += __shfl_xor(v[i][j], off, kOneElLanes);
-      if ((i * NB + j) % kOneElLanes != part) continue;
-      if (a.S) { a.S[mu * n + nu] = f * s[i][j]; a.S[nu * n + mu] = f * s[i][j]; }
-      if (a.T) { a.T[mu * n + nu] = f * t[i][j]; a.T[nu * n + mu] = f * t[i][j]; }
-      if (a.V) { a.V[mu * n + nu] = f * v[i][j]; a.V[nu * n + mu] = f * v[i][j]; }
-    }
+        for (int off = kOneElLanes / 2; off > 0; off >>= 1)
+          v[i][j] += __shfl_xor(v[i][j], off, kOneElLanes);
+        if ((i * NB + j) % kOneElLanes != part) continue;
+        if (a.S) { a.S[mu * n + nu] = f * s[i][j]; a.S[nu * n + mu] = f * s[i][j]; }
+        if (a.T) { a.T[mu * n + nu] = f * t[i][j]; a.T[nu * n + mu] = f * t[i][j]; }
+        if (a.V) { a.V[mu * n + nu] = f * v[i][j]; a.V[nu * n + mu] = f * v[i][j]; }
+      }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -602,9 +603,9 @@ hipError_t one_electron_grad_launch(const OneElGradArgs& a, hipStream_t s) {
 template <int LA, int LB>
 hipError_t one_electron_class(const OneElArgs& a, hipStream_t s) {
   const int c = 3 * LA + LB;
-  const int cnt = a.cls_begin[c + 1] - a.cls_begin[c];
+  const long long cnt = a.cls_begin[c + 1] - a.cls_begin[c];
   if (cnt <= 0) return hipSuccess;
-  hipLaunchKernelGGL((one_electron_kernel<LA, LB>), dim3((cnt * kOneElLanes + kOneElBlock - 1) / kOneElBlock),
+  hipLaunchKernelGGL((one_electron_kernel<LA, LB>), dim3(static_cast<unsigned>(one_el_blocks(cnt))),
                      dim3(kOneElBlock), 0, s, a);
   return hipGetLastError();
 }
