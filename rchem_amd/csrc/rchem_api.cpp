@@ -23,6 +23,7 @@
 
 #include "../../include/rchem_gpu.h"
 #include "boys.hpp"
+#include "tile_width.hpp"
 #include "types.hpp"
 
 namespace rchem {
@@ -381,6 +382,7 @@ struct rchem_ctx {
 
   // tiles for a threshold
   double tiles_tau = -1.0;
+  int tiles_use = 0;  // TileUse
   std::vector<Tile> tiles;
   std::vector<QClass> qclasses;   // device-planner classes
   std::vector<QClass> hclasses;   // classes of the host-built tile list (tensor, gradient)
@@ -1098,14 +1100,6 @@ void class_ls(int X, int* l1, int* l2) {
       }
 }
 
-// Lanes to a quartet of the tensor and Schwarz kernels: at most 8, and no more
-// than give the class (a bucket of it) 8 waves to a SIMD.  A lane's chain of
-// primitive quartets was the time of a small tensor's kernels: (H2O)_3 6-31G
-// (ss|ss) 0.289 -> 0.080 ms, all classes 0.89 -> 0.23, the call 2.35 -> 1.66; of
-// the bounds of (H2O)_8, (ss|ss) and (ps|ps): 0.42 and 0.14 -> 0.07 and 0.03 ms.
-constexpr int kTensorMaxShift = 3;
-constexpr double kTensorWaves = 8192.0;
-
 // Schwarz bounds for every shell pair (exact Boys), once per basis.
 int compute_schwarz(rchem_ctx* ctx) {
   if (ctx->have_schwarz) return RCHEM_OK;
@@ -1132,10 +1126,8 @@ int compute_schwarz(rchem_ctx* ctx) {
     ClassKernel k;
     TRY(class_kernel(ctx, l1, l2, l1, l2, kModeDiag, kBoysExact, 0, &k));
     for (const Bucket& bk : ctx->buckets[X]) {
-      int sh = 0;
-      while (k.fn && sh < kTensorMaxShift && (2 << sh) <= bk.np &&
-             (bk.end - bk.begin) / 64.0 * (2 << sh) <= kTensorWaves)
-        ++sh;
+      const int sh = tile_shift(k.fn ? TileEngine::kLanes : TileEngine::kLane,
+                                (bk.end - bk.begin) / 64.0, bk.np);
       const int w = 64 >> sh;
       for (int j = bk.begin; j < bk.end; j += w)
         ctx->tiles.push_back(Tile{-1, j, std::min(w, bk.end - j), sh});
@@ -1273,11 +1265,16 @@ double per_prim_flops(const QClass& qc, int* hrr) {
   return fv + 68.0 + 4.0 * (qc.la + qc.lb + qc.lc + qc.ld);
 }
 
-// Host-built tile list (used for the dense tensor, where tau = 0 and systems
-// are small).
-int prepare_host_tiles(rchem_ctx* ctx, double tau) {
+// What a host-built tile list is for: the widths of its tiles go by the kernels
+// that take them.
+enum TileUse { kTilesTensor, kTilesGradient };
+
+// Host-built tile list, of the dense tensor (tau = 0) or of the gradient's
+// derivative quartets.
+int prepare_host_tiles(rchem_ctx* ctx, double tau, TileUse use) {
   TRY(prepare_pairs(ctx, tau));
-  if (ctx->tiles_tau == tau) return RCHEM_OK;
+  if (ctx->tiles_tau == tau && ctx->tiles_use == use) return RCHEM_OK;
+  ctx->tiles_tau = -1.0;
   ctx->tiles.clear();
   ctx->hclasses.clear();
   int curX = -1, curY = -1;
@@ -1286,24 +1283,26 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
     qc.ntiles = static_cast<int>(ctx->tiles.size()) - qc.tile_begin;
     if (curX >= 0 && qc.ntiles > 0) ctx->hclasses.push_back(qc);
   };
-  // 1 << sh lanes to a quartet where a class's tiles are too few for the chip
   std::vector<double> waves(kNumPairClasses * kNumPairClasses, 0.0);
-  std::vector<int> most(waves.size(), 0);
+  std::vector<TileEngine> engine(waves.size(), TileEngine::kLane);
   for_each_task(ctx, tau, [&](int X, int Y, int, int, int lo, int hi) {
     waves[X * kNumPairClasses + Y] += (hi - lo + 63) / 64;
   });
-  int rc = RCHEM_OK;
   for (int X = 0; X < kNumPairClasses; ++X)
-    for (int Y = 0; Y < kNumPairClasses && rc == RCHEM_OK; ++Y) {
+    for (int Y = 0; Y < kNumPairClasses; ++Y) {
       const int c = X * kNumPairClasses + Y;
       if (waves[c] == 0.0) continue;
       const QClass q = make_qclass(X, Y);
-      ClassKernel fn;
-      rc = class_kernel(ctx, q.la, q.lb, q.lc, q.ld, kModeTensor, kBoysExact, 0, &fn);
-      if (!fn.fn) continue;  // the other engines spread a quartet over a wave
-      while (most[c] < kTensorMaxShift && waves[c] * (2 << most[c]) <= kTensorWaves) ++most[c];
+      if (use == kTilesGradient) {
+        const bool lane = !ctx->force_generic && eri_grad_launcher(q.la, q.lb, q.lc, q.ld);
+        engine[c] = lane ? TileEngine::kLane : TileEngine::kWave;
+      } else {
+        ClassKernel fn;
+        TRY(class_kernel(ctx, q.la, q.lb, q.lc, q.ld, kModeTensor, kBoysExact, 0, &fn));
+        // the other engines spread a quartet over a wave
+        engine[c] = fn.fn ? TileEngine::kLanes : TileEngine::kLane;
+      }
     }
-  TRY(rc);
   for_each_task(ctx, tau, [&](int X, int Y, int i, int b, int lo, int hi) {
     if (X != curX || Y != curY) {
       flush();
@@ -1312,8 +1311,8 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
       qc = make_qclass(X, Y);
       qc.tile_begin = static_cast<int>(ctx->tiles.size());
     }
-    int sh = most[X * kNumPairClasses + Y];
-    while (sh > 0 && (1 << sh) > ctx->buckets[Y][b].np) --sh;
+    const int c = X * kNumPairClasses + Y;
+    const int sh = tile_shift(engine[c], waves[c], ctx->buckets[Y][b].np);
     const int w = 64 >> sh;
     for (int j = lo; j < hi; j += w) ctx->tiles.push_back(Tile{i, j, std::min(w, hi - j), sh});
   });
@@ -1327,6 +1326,7 @@ int prepare_host_tiles(rchem_ctx* ctx, double tau) {
   }
   TRY(upload_tiles(ctx));
   ctx->tiles_tau = tau;
+  ctx->tiles_use = use;
   return RCHEM_OK;
 }
 
@@ -2479,7 +2479,7 @@ int rchem_eri_tensor(rchem_ctx* ctx, double* I, const rchem_opts* opts) {
   const size_t n = static_cast<size_t>(ctx->nbf);
   const size_t n4 = n * n * n * n;
   if (n > 200) return ctx->fail(RCHEM_ERR_INVALID, "tensor too large (nbf > 200)");
-  TRY(prepare_host_tiles(ctx, 0.0));
+  TRY(prepare_host_tiles(ctx, 0.0, kTilesTensor));
   DevBuf t;
   HIPC(t.ensure(n4 * sizeof(double)));
   HIPC(fill_launch(t.as<double>(), n4, 0.0, ctx->stream));
@@ -3957,7 +3957,7 @@ int rchem_rhf_gradient(rchem_ctx* ctx, int natom, const double* Z, const double*
   // two-electron part: derivative quartets contracted with Gamma on the fly
   const double tau = std::min(opts->jk.schwarz_thresh > 0.0 ? opts->jk.schwarz_thresh : 1e-12,
                               1e-12) * 1e-2;
-  TRY(prepare_host_tiles(ctx, tau));
+  TRY(prepare_host_tiles(ctx, tau, kTilesGradient));
   std::vector<int2> pat(ctx->pairs.size());
   for (size_t i = 0; i < pat.size(); ++i)
     pat[i] = make_int2(satom[ctx->pair_shells[i].first], satom[ctx->pair_shells[i].second]);
