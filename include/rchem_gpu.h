@@ -252,13 +252,12 @@ typedef struct rchem_scf_opts {
   int purify;          /* 1: each iteration's density D = X P X^T with P, the projector
                           onto the nocc lowest eigenvectors of F' = X^T F X, from
                           purification (products only) instead of the
-                          eigensolver, which takes over only an iteration whose F'
-                          has no gap.  Single-molecule SCF and gradient (whose
-                          energy-weighted density is W = D F D either way); the
-                          batched SCF ignores it.  0 (default): the projector of
-                          rchem's eigh every iteration (rchem.rs:74-78), which
-                          matrices of up to 1024 functions too form by products
-                          where F' has a gap */
+                          eigensolver, which takes over where F' has no gap (until
+                          its eigenvalues show one).  Single-molecule SCF and gradient
+                          (whose energy-weighted density is W = D F D either way).  0
+                          (default): rchem's eigh every iteration (rchem.rs:74-78).  The
+                          batched SCF ignores it: its molecules' projectors are formed
+                          by products where the largest has at most 128 functions */
   double damping;      /* a in [0, 1): each new density is mixed with the previous one,
                           D <- (1 - a) D_new + a D_old (a convergence aid for hard
                           cases; the converged density is the same stationary point);

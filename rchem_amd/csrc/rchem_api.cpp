@@ -2799,6 +2799,14 @@ struct FockGraph {
   }
 };
 
+// Whether a purification of a matrix with the n eigenvalues w (ascending) is
+// worth trying.  A step gains a factor of 1.2 to 2 on the gap, and Gershgorin's
+// interval, which it starts from, is several times the spectrum: a gap of 1e-6 of
+// the spectrum takes about 90 steps, where the kernels stop at 100 or 200.
+bool purifiable(const double* w, int n, int nocc) {
+  return nocc <= 0 || nocc >= n || w[nocc] - w[nocc - 1] > 1e-6 * (w[n - 1] - w[0]);
+}
+
 int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
             const rchem_scf_opts* opts, rchem_scf_result* res, double dconv) {
   if (!ctx) return RCHEM_ERR_INVALID;
@@ -2843,33 +2851,31 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
   // kPurifyMax steps (no gap at the Fermi level), and the eigensolver takes over.
   constexpr int kPurifyMax = 200;
   constexpr double kPurifyTol = 1e-9;
-  // Up to kDensityMaxN functions the whole density, F' and projector included,
-  // is one launch (scf_density.hip); it reads as a purification of kSmallSteps
-  // steps that converged in the first or not at all.
-  const bool small = n <= kDensityMaxN;
+  // With opts->purify, up to kDensityMaxN functions the whole density, F' and
+  // projector included, is one launch (scf_density.hip); it reads as a
+  // purification of kSmallSteps steps that converged in the first or not at all.
+  const bool small = opts->purify && n <= kDensityMaxN;
   constexpr int kSmallSteps = 3;
   DevBuf dflag;
   HIPC(dflag.ensure(sizeof(double) * 2 * kSmallSteps));
   if (small) HIPC(fill_launch(dflag.as<double>(), 2 * kSmallSteps, 1.0, ctx->stream));
   DevBuf dP, dP2, dP3, dpl, dph, dpar, dsp2;
   // above that, up to kSp2MaxN (where the library's products on the whole chip
-  // become the better ones), the same scheme takes one launch to a step, for
-  // either value of opts->purify; a matrix without a gap takes the eigensolver
+  // become the better ones), a step is one launch
   constexpr int kSp2MaxN = 1024;
-  const bool sp2 = !small && n <= kSp2MaxN && opts->nocc < n;
-  if (sp2) {
-    const size_t wd = sp2_workspace(n, kPurifyMax);
-    HIPC(dsp2.ensure(wd * sizeof(double)));
-    HIPC(fill_launch(dsp2.as<double>(), wd, 0.0, ctx->stream));
+  const bool sp2 = opts->purify && !small && n <= kSp2MaxN && opts->nocc < n;
+  if (opts->purify && !small) {
     HIPC(dP.ensure(n2 * sizeof(double)));
     HIPC(dpl.ensure(n * sizeof(double)));
     HIPC(dph.ensure(n * sizeof(double)));
     HIPC(dpar.ensure((4 + 2 * kPurifyMax) * sizeof(double)));
-  } else if (opts->purify) {
-    for (DevBuf* b : {&dP, &dP2, &dP3}) HIPC(b->ensure(n2 * sizeof(double)));
-    HIPC(dpl.ensure(n * sizeof(double)));
-    HIPC(dph.ensure(n * sizeof(double)));
-    HIPC(dpar.ensure((4 + 2 * kPurifyMax) * sizeof(double)));
+    if (sp2) {
+      const size_t wd = sp2_workspace(n, kPurifyMax);
+      HIPC(dsp2.ensure(wd * sizeof(double)));
+      HIPC(fill_launch(dsp2.as<double>(), wd, 0.0, ctx->stream));
+    } else {
+      for (DevBuf* b : {&dP2, &dP3}) HIPC(b->ensure(n2 * sizeof(double)));
+    }
   }
   auto purify_step = [&](double* coef) -> int {
     BLASC(rocblas_dgemm(hb, rocblas_operation_none, rocblas_operation_none, n, n, n, &one,
@@ -2955,29 +2961,30 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
     return RCHEM_OK;
   };
   // Dout = the density of Fm: F' = X^T F X, eigh, C = X C', D = C_occ C_occ^T
-  // (rchem.rs:56-59, 74-78, 101-104), or X P X^T by purification; *psteps
-  // (may be null) receives the purification's step count, 0 if the
-  // eigensolver formed it
+  // (rchem.rs:56-59, 74-78, 101-104), or with opts->purify X P X^T by
+  // purification; *psteps (may be null) receives the purification's step count,
+  // 0 if the eigensolver formed it.  A purification that failed is not tried
+  // again before the eigenvalues show a gap.
+  bool purifying = opts->purify != 0;
   auto density = [&](const double* Fm, double* Dout, int* psteps) -> int {
     if (psteps) *psteps = 0;
-    if (small) {
+    if (purifying && small) {
       HIPC(density_small_launch(Fm, dX.as<double>(), n, n, nullptr, opts->nocc, nullptr, 1, Dout,
                                 dflag.as<double>(), ctx->stream));
       double f[2] = {0.0, 1.0};
       HIPC(hipMemcpyAsync(f, dflag.p, sizeof(f), hipMemcpyDeviceToHost, ctx->stream));
       HIPC(hipStreamSynchronize(ctx->stream));
       if (f[1] == 0.0) {
-        if (psteps && opts->purify) *psteps = kSmallSteps;
+        if (psteps) *psteps = kSmallSteps;
         return RCHEM_OK;
       }
-      // no gap: the purification in memory (if asked for) and the eigensolver
     }
     TRY(orthogonalise(Fm));
-    if (opts->purify || sp2) {
+    if (purifying && !small) {
       int steps = 0;
       TRY(purify(&steps));
       if (steps > 0) {
-        if (psteps && opts->purify) *psteps = steps;
+        if (psteps) *psteps = steps;
         return density_from_p(Dout);
       }
     }
@@ -2988,6 +2995,12 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
     BLASC(rocblas_dgemm(hb, rocblas_operation_none, rocblas_operation_transpose, n, n,
                         opts->nocc, &one, dC.as<double>(), n, dC.as<double>(), n, &zero, Dout,
                         n));
+    if (opts->purify && opts->nocc < n) {
+      std::vector<double> w(n);
+      HIPC(hipMemcpyAsync(w.data(), dw.p, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+      HIPC(hipStreamSynchronize(ctx->stream));
+      purifying = purifiable(w.data(), n, opts->nocc);
+    }
     return RCHEM_OK;
   };
   auto energy = [&](const double* Fm, double* e) -> int {
