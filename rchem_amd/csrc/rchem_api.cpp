@@ -3490,11 +3490,13 @@ int batch_chunk(rchem_ctx* ctx, int m0, int m1, const int* natom, const int* Z,
   HIPC(hipMemcpyAsync(df0.p, f0.data(), sizeof(int) * B, hipMemcpyHostToDevice, st));
   HIPC(hipMemcpyAsync(dnb.p, nb.data(), sizeof(int) * B, hipMemcpyHostToDevice, st));
   HIPC(hipMemcpyAsync(dnocc.p, nocc.data(), sizeof(int) * B, hipMemcpyHostToDevice, st));
-  auto gemm_b = [&](rocblas_operation ta, rocblas_operation tb, const double* A, const double* Bm,
-                    double* C) {
+  auto gemm_n = [&](rocblas_operation ta, rocblas_operation tb, const double* A, const double* Bm,
+                    double* C, int count) {
     return rocblas_dgemm_strided_batched(hb, ta, tb, nm, nm, nm, &one, A, nm, sm, Bm, nm, sm,
-                                         &zero, C, nm, sm, Bs);
+                                         &zero, C, nm, sm, count);
   };
+  auto gemm_b = [&](rocblas_operation ta, rocblas_operation tb, const double* A, const double* Bm,
+                    double* C) { return gemm_n(ta, tb, A, Bm, C, Bs); };
   // Loewdin X_b = U_b lambda_b^-1/2 U_b^T (rchem.rs:44-51), padding = identity
   HIPC(batch_pack(dS.as<double>(), n, df0.as<int>(), dnb.as<int>(), nm, Bs, 1.0, dSp.as<double>(), st));
   HIPC(hipMemcpyAsync(dT1.p, dSp.p, sizeof(double) * m2 * Bs, hipMemcpyDeviceToDevice, st));
@@ -3506,38 +3508,88 @@ int batch_chunk(rchem_ctx* ctx, int m0, int m1, const int* natom, const int* Z,
                dT1.as<double>(), dX.as<double>()));
   HIPC(hipStreamSynchronize(st));
   dS.release();  // its blocks live on in dSp
-  // density from a padded Fock batch: F' = X^T F X, eigh, C = X C', D = C_occ C_occ^T
-  DevBuf dflag;
-  HIPC(dflag.ensure(sizeof(double) * 2 * B));
-  std::vector<double> flags(2 * static_cast<size_t>(B));
-  auto density_b = [&](const double* Fb) -> int {
-    if (nm <= kDensityMaxN) {
-      // every molecule's in one launch, unless one of them has no gap
-      HIPC(density_small_launch(Fb, dX.as<double>(), nm, nm, dnb.as<int>(), 0, dnocc.as<int>(), Bs,
-                                dDb.as<double>(), dflag.as<double>(), st));
-      HIPC(hipMemcpyAsync(flags.data(), dflag.p, sizeof(double) * 2 * Bs, hipMemcpyDeviceToHost,
-                          st));
-      HIPC(hipStreamSynchronize(st));
-      bool good = true;
-      for (int s = 0; s < Bs; ++s) good = good && flags[2 * s + 1] == 0.0;
-      if (good) {
-        HIPC(batch_unpack(dDb.as<double>(), nm, df0.as<int>(), dnb.as<int>(), Bs, n,
-                          dD.as<double>(), st));
-        return RCHEM_OK;
-      }
-    }
-    BLASC(gemm_b(rocblas_operation_none, rocblas_operation_none, Fb, dX.as<double>(), dT1.as<double>()));
-    BLASC(gemm_b(rocblas_operation_transpose, rocblas_operation_none, dX.as<double>(),
-                 dT1.as<double>(), dW.as<double>()));
+  // Densities of `count` slots from padded Fock matrices by the eigensolver:
+  // F' = X^T F X, eigh, C = X C', D = C_occ C_occ^T into out
+  auto eigen_b = [&](const double* Fb, const double* Xb, const int* noccb, int count,
+                     double* out) -> int {
+    BLASC(gemm_n(rocblas_operation_none, rocblas_operation_none, Fb, Xb, dT1.as<double>(), count));
+    BLASC(gemm_n(rocblas_operation_transpose, rocblas_operation_none, Xb, dT1.as<double>(),
+                 dW.as<double>(), count));
     BLASC(rocsolver_dsyevd_strided_batched(hb, rocblas_evect_original, rocblas_fill_upper, nm,
                                            dW.as<double>(), nm, sm, dw.as<double>(), nm,
-                                           de.as<double>(), nm, dinfo.as<rocblas_int>(), Bs));
-    BLASC(gemm_b(rocblas_operation_none, rocblas_operation_none, dX.as<double>(), dW.as<double>(),
-                 dC.as<double>()));
-    HIPC(batch_mask_cols(dC.as<double>(), nm, dnocc.as<int>(), Bs, st));
-    BLASC(gemm_b(rocblas_operation_none, rocblas_operation_transpose, dC.as<double>(),
-                 dC.as<double>(), dDb.as<double>()));
-    HIPC(batch_unpack(dDb.as<double>(), nm, df0.as<int>(), dnb.as<int>(), Bs, n, dD.as<double>(), st));
+                                           de.as<double>(), nm, dinfo.as<rocblas_int>(), count));
+    BLASC(gemm_n(rocblas_operation_none, rocblas_operation_none, Xb, dW.as<double>(),
+                 dC.as<double>(), count));
+    HIPC(batch_mask_cols(dC.as<double>(), nm, noccb, count, st));
+    BLASC(gemm_n(rocblas_operation_none, rocblas_operation_transpose, dC.as<double>(),
+                 dC.as<double>(), out, count));
+    return RCHEM_OK;
+  };
+  // The densities of a padded Fock batch.  Up to kDensityMaxN functions all the
+  // molecules' in one launch; those whose F' has no gap are gathered for the
+  // eigensolver, and left out of the products until their eigenvalues show one.
+  DevBuf dflag, dtry, deig, dFg, dXg;  // deig: f0, nb, nocc and slot of the gathered ones
+  HIPC(dflag.ensure(sizeof(double) * 2 * B));
+  std::vector<double> flags(2 * static_cast<size_t>(B)), weig;
+  std::vector<char> no_gap(B, 0);  // per molecule
+  auto density_b = [&](const double* Fb) -> int {
+    if (nm > kDensityMaxN) {
+      TRY(eigen_b(Fb, dX.as<double>(), dnocc.as<int>(), Bs, dDb.as<double>()));
+      HIPC(batch_unpack(dDb.as<double>(), nm, df0.as<int>(), dnb.as<int>(), Bs, n, dD.as<double>(),
+                        st));
+      return RCHEM_OK;
+    }
+    std::vector<int> occ(Bs);  // -1: not tried
+    for (int s = 0; s < Bs; ++s) occ[s] = no_gap[slot_mol[s]] ? -1 : nocc[slot_mol[s]];
+    const bool left_out = std::count(occ.begin(), occ.end(), -1) > 0;
+    if (left_out) {
+      HIPC(dtry.ensure(sizeof(int) * Bs));
+      HIPC(hipMemcpyAsync(dtry.p, occ.data(), sizeof(int) * Bs, hipMemcpyHostToDevice, st));
+    }
+    HIPC(density_small_launch(Fb, dX.as<double>(), nm, nm, dnb.as<int>(), 0,
+                              left_out ? dtry.as<int>() : dnocc.as<int>(), Bs, dDb.as<double>(),
+                              dflag.as<double>(), st));
+    HIPC(hipMemcpyAsync(flags.data(), dflag.p, sizeof(double) * 2 * Bs, hipMemcpyDeviceToHost, st));
+    HIPC(hipStreamSynchronize(st));
+    std::vector<int> gathered;  // f0, nb, nocc, slot of each
+    for (int s = 0; s < Bs; ++s)
+      if (flags[2 * s + 1] != 0.0) gathered.push_back(s);
+    // (the gathered ones' blocks of dDb are not densities; theirs follow)
+    HIPC(batch_unpack(dDb.as<double>(), nm, df0.as<int>(), dnb.as<int>(), Bs, n, dD.as<double>(),
+                      st));
+    const int ng = static_cast<int>(gathered.size());
+    if (ng == 0) return RCHEM_OK;
+    const std::vector<int> slots(gathered);
+    gathered.resize(4 * static_cast<size_t>(ng));
+    for (int g = 0; g < ng; ++g) {
+      const int b = slot_mol[slots[g]];
+      gathered[g] = f0[b];
+      gathered[ng + g] = nb[b];
+      gathered[2 * ng + g] = nocc[b];
+      gathered[3 * ng + g] = slots[g];
+    }
+    HIPC(deig.ensure(sizeof(int) * gathered.size()));
+    HIPC(dFg.ensure(sizeof(double) * m2 * ng));
+    HIPC(dXg.ensure(sizeof(double) * m2 * ng));
+    HIPC(hipMemcpyAsync(deig.p, gathered.data(), sizeof(int) * gathered.size(),
+                        hipMemcpyHostToDevice, st));
+    const int* const dslot = deig.as<int>() + 3 * ng;
+    HIPC(batch_gather(Fb, m2 * Bs, nm, dslot, ng, 1, dFg.as<double>(), m2 * ng, nm, st));
+    HIPC(batch_gather(dX.as<double>(), m2 * Bs, nm, dslot, ng, 1, dXg.as<double>(), m2 * ng, nm,
+                      st));
+    TRY(eigen_b(dFg.as<double>(), dXg.as<double>(), deig.as<int>() + 2 * ng, ng,
+                dDb.as<double>()));
+    HIPC(batch_unpack(dDb.as<double>(), nm, deig.as<int>(), deig.as<int>() + ng, ng, n,
+                      dD.as<double>(), st));
+    weig.resize(static_cast<size_t>(nm) * ng);
+    HIPC(hipMemcpyAsync(weig.data(), dw.p, sizeof(double) * weig.size(), hipMemcpyDeviceToHost,
+                        st));
+    HIPC(hipStreamSynchronize(st));
+    // (a block's padding has the largest eigenvalues)
+    for (int g = 0; g < ng; ++g) {
+      const int b = slot_mol[slots[g]];
+      no_gap[b] = !purifiable(weig.data() + static_cast<size_t>(nm) * g, nb[b], nocc[b]);
+    }
     return RCHEM_OK;
   };
   auto density_dense = [&](const double* Fd) -> int {

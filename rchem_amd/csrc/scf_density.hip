@@ -80,8 +80,8 @@ __device__ __forceinline__ void triangle(int t, int* i, int* j) {
 // Matrix m: F + m f_stride, X + m x_stride, D + m d_stride with leading
 // dimension ld, size nb[m] (n where nb is null) and nocc[m] (nocc1 where null).
 // flag[2m + 1]: 0 once D holds the density, 1 if the purification has not
-// converged (flag[2m] is 0.5: the pair reads as a purification step's
-// coefficient and tr(P - P^2)).
+// converged or was not asked for (nocc < 0) (flag[2m] is 0.5: the pair reads as a
+// purification step's coefficient and tr(P - P^2)).
 __global__ __launch_bounds__(64 * kMaxWaves) void density_small_kernel(
     const double* __restrict__ Fb, const double* __restrict__ Xb, size_t stride, int ld, int n0,
     const int* __restrict__ nb, int nocc1, const int* __restrict__ noccb, double* __restrict__ Db,
@@ -90,6 +90,13 @@ __global__ __launch_bounds__(64 * kMaxWaves) void density_small_kernel(
   __shared__ double red[2 * kMaxWaves];
   const int m = blockIdx.x;
   const int n = nb ? nb[m] : n0, nocc = noccb ? noccb[m] : nocc1;
+  if (nocc < 0) {  // block-uniform
+    if (threadIdx.x == 0) {
+      flag[2 * m] = 0.5;
+      flag[2 * m + 1] = 1.0;
+    }
+    return;
+  }
   const double* __restrict__ F = Fb + m * stride;
   const double* __restrict__ X = Xb + m * stride;
   double* __restrict__ D = Db + m * stride;
