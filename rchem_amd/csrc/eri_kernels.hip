@@ -13,7 +13,8 @@ namespace rchem {
 using EriLaunchFn = hipError_t (*)(const EriArgs&, int, hipStream_t);
 struct EriPart {
   hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
-  size_t (*slab)(int cus) = nullptr;
+  size_t slab = 0;
+  int groups = 0;
   bool (*rows_fit)(int kw) = nullptr;
 };
 

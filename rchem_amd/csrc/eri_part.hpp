@@ -311,17 +311,15 @@ __global__ __launch_bounds__(THREADS, MINW) void eri_part_kernel(
   }
 }
 
-// Workgroups a compute unit can hold by registers, and the bytes of the slabs of
-// a launch with as many.
+// Workgroups a compute unit can hold by registers, and the bytes of one's slab.
 template <int LA, int LB, int LC, int LD>
-constexpr int part_groups() {
+constexpr int eri_part_groups() {
   using C = EriParts<LA, LB, LC, LD>;
   return 4 * C::MINW / C::W;
 }
 template <int LA, int LB, int LC, int LD>
-size_t eri_part_slab(int cus) {
-  return static_cast<size_t>(cus) * part_groups<LA, LB, LC, LD>() *
-         EriClass<LA, LB, LC, LD>::NACC * 64 * sizeof(double);
+constexpr size_t eri_part_slab() {
+  return EriClass<LA, LB, LC, LD>::NACC * 64 * sizeof(double);
 }
 
 template <int LA, int LB, int LC, int LD, int ROWS>
@@ -349,19 +347,23 @@ bool eri_part_rows_fit(int kw) {
 template <int LA, int LB, int LC, int LD>
 hipError_t eri_part_launch(const EriArgs& a, double* slab, size_t bytes, int cus, hipStream_t s) {
   constexpr int NA = ncart(LA), NB = ncart(LB);
-  constexpr int groups = part_groups<LA, LB, LC, LD>();
-  if (!a.Dp || !a.Jp || !slab || eri_part_slab<LA, LB, LC, LD>(cus) > bytes)
-    return hipErrorInvalidValue;
+  constexpr int groups = eri_part_groups<LA, LB, LC, LD>();
+  // no more workgroups than the slab was reserved for
+  const size_t most = bytes / eri_part_slab<LA, LB, LC, LD>();
+  if (!a.Dp || !a.Jp || !slab || most == 0) return hipErrorInvalidValue;
   const size_t fixed = eri_part_fixed<LA, LB, LC, LD>();
   const size_t rows = sizeof(double) * (NA + NB) * static_cast<size_t>(a.kw);
   // K rows in LDS where they fit, the density's too unless that costs a workgroup
   const auto held = [&](size_t lds) { return std::min<int>(groups, kLdsPerCu / lds); };
+  const auto grid = [&](int n) {
+    return static_cast<int>(std::min(most, static_cast<size_t>(n) * cus));
+  };
   const int rows2 = held(fixed + 2 * rows), rows1 = held(fixed + rows);
   if (a.chunk_range && rows2 > 0 && rows2 == rows1)
-    return eri_part_launch_rows<LA, LB, LC, LD, 2>(a, slab, fixed + 2 * rows, rows2 * cus, s);
+    return eri_part_launch_rows<LA, LB, LC, LD, 2>(a, slab, fixed + 2 * rows, grid(rows2), s);
   if (a.chunk_range && rows1 > 0)
-    return eri_part_launch_rows<LA, LB, LC, LD, 1>(a, slab, fixed + rows, rows1 * cus, s);
-  return eri_part_launch_rows<LA, LB, LC, LD, 0>(a, slab, fixed, held(fixed) * cus, s);
+    return eri_part_launch_rows<LA, LB, LC, LD, 1>(a, slab, fixed + rows, grid(rows1), s);
+  return eri_part_launch_rows<LA, LB, LC, LD, 0>(a, slab, fixed, grid(held(fixed)), s);
 }
 
 }  // namespace rchem

@@ -483,7 +483,8 @@ def part_tu_source(key):
         f"hipError_t eri_part_launch_c{key}(const EriArgs& a, double* slab, size_t bytes, int cus,",
         "                                    hipStream_t s) {",
         f"  return eri_part_launch<{A}>(a, slab, bytes, cus, s);", "}",
-        f"size_t eri_part_slab_c{key}(int cus) {{ return eri_part_slab<{A}>(cus); }}",
+        f"size_t eri_part_slab_c{key}() {{ return eri_part_slab<{A}>(); }}",
+        f"int eri_part_groups_c{key}() {{ return eri_part_groups<{A}>(); }}",
         f"bool eri_part_rows_c{key}(int kw) {{ return eri_part_rows_fit<{A}>(kw); }}", "",
         "}  // namespace rchem", ""])
 
@@ -728,14 +729,14 @@ def main():
                     f"return eri_stream_launcher_c{k}(mode);")
     disp += ["  return nullptr;", "}", ""]
     disp += [f"hipError_t eri_part_launch_c{k}(const EriArgs&, double*, size_t, int, hipStream_t);\n"
-             f"size_t eri_part_slab_c{k}(int);\nbool eri_part_rows_c{k}(int);"
+             f"size_t eri_part_slab_c{k}();\nint eri_part_groups_c{k}();\nbool eri_part_rows_c{k}(int);"
              for k in PART_SHAPES]
     disp += ["", "// Partwise Fock-build kernel of the class (exact Boys, FP64); null if none.",
              "EriPart eri_part_launcher(int la, int lb, int lc, int ld) {"]
     for k in PART_SHAPES:
         disp.append(f"  if (la == {k[0]} && lb == {k[1]} && lc == {k[2]} && ld == {k[3]}) "
-                    f"return EriPart{{eri_part_launch_c{k}, eri_part_slab_c{k}, "
-                    f"eri_part_rows_c{k}}};")
+                    f"return EriPart{{eri_part_launch_c{k}, eri_part_slab_c{k}(), "
+                    f"eri_part_groups_c{k}(), eri_part_rows_c{k}}};")
     disp += ["  return EriPart{};", "}", ""]
     write_if_changed(os.path.join(out_dir, "eri_dispatch.inc"), "\n".join(disp))
     write_if_changed(os.path.join(out_dir, "flops_per_class.json"),

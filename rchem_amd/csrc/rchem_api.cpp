@@ -44,12 +44,13 @@ hipError_t begin_launch(double* J, double* K, size_t n2, double* stats, size_t n
 hipError_t plan_launch(const PlanArgs& a, const PlanBuffers& b, hipStream_t s);
 EriLaunchFn eri_jk_lds_launcher(int la, int lb, int lc, int ld, int bm, int fp32, int v);
 EriStreamFn eri_stream_launcher(int la, int lb, int lc, int ld, int mode);
-// Partwise Fock-build kernel of a class: its launcher and the bytes of global
-// memory its workgroups keep a tile's accumulators in, and whether the K rows of
-// kw columns fit the LDS.
+// Partwise Fock-build kernel of a class: its launcher, the bytes of global memory
+// a workgroup keeps a tile's accumulators in, the workgroups a compute unit holds,
+// and whether the K rows of kw columns fit the LDS.
 struct EriPart {
   hipError_t (*launch)(const EriArgs&, double* slab, size_t bytes, int cus, hipStream_t) = nullptr;
-  size_t (*slab)(int cus) = nullptr;
+  size_t slab = 0;
+  int groups = 0;
   bool (*rows_fit)(int kw) = nullptr;
 };
 EriPart eri_part_launcher(int la, int lb, int lc, int ld);
@@ -1412,17 +1413,14 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   // Split tiles (PrimSplit) where a class's longest tile is longer than its
   // waves' share of the class; the tiles reserved are then counted again.
   std::vector<int> limit(nq, 0);
-  std::vector<char> partwise(nq, 0);
+  std::vector<EriPart> partwise(nq);
   bool split = false;
   for (size_t c = 0; c < nq; ++c) {
     const QClass& qc = ctx->qclasses[c];
     ClassKernel k;
     if (qc.quartets > 0)
       TRY(class_kernel(ctx, qc.la, qc.lb, qc.lc, qc.ld, kModeJK, kBoysExact, 0, &k));
-    if (k.part.launch) {
-      HIPC(ctx->part_slab_d.ensure(k.part.slab(ctx->cus)));
-      partwise[c] = 1;
-    }
+    partwise[c] = k.part;
     if (!k.fn) continue;  // the other engines spread a quartet over a wave
     limit[c] = split_limit(qc, iters[c]);
     if (limit[c] >= npmax[c]) limit[c] = 0;
@@ -1458,15 +1456,19 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   }
   // chunks short enough that a class has some thousand of them
   std::vector<int> chunk_most(nq);
+  size_t slab = 0;  // of the class that needs most, for no more workgroups than tiles
   for (size_t c = 0; c < nq; ++c) {
     double tiles = 0.0;
     for (const double x : bra_cap[c]) tiles += x;
-    if (partwise[c]) {  // a chunk to a workgroup, one workgroup a CU
+    if (partwise[c].launch) {  // a chunk to a workgroup, one workgroup a CU
       chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(4.0, tiles / (16.0 * ctx->cus))));
+      slab = std::max(slab, partwise[c].slab * static_cast<size_t>(std::max(
+                                1.0, std::min(tiles, 1.0 * ctx->cus * partwise[c].groups))));
       continue;
     }
     chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(8.0, tiles / kMinChunks)));
   }
+  if (slab > 0) HIPC(ctx->part_slab_d.ensure(slab));
   // segments and passes
   rchem_ctx::Pass cur{0, 0, 0, 0, 0, 0, 0};
   double pass_cap = 0.0, pass_ccap = 0.0;
