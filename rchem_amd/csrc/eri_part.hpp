@@ -27,6 +27,10 @@
 // (dp|pp) 17.6, 15.5; (dp|dp) 68.6, 16.2; (dd|ds) 20.5, 8.9; (dd|pp) 42.0, 8.6;
 // (dd|dp) 55.0, 18.1; (dd|dd) 32.0, 6.9.  The build: 271 -> 133, and 127 with the
 // chunks handed out by a counter.
+//
+// A tile is one lane's chain of primitive quartets, so where a class has fewer
+// tiles than the chip workgroups they are split over the primitives as in the
+// per-lane kernels (PrimSplit, part_split_limit).
 // The recurrences are chgp.c:412-586 (VRR) and chgp.c:44-135 (HRR).
 #pragma once
 #include "eri_common.hpp"
@@ -60,13 +64,20 @@ __device__ __forceinline__ void part_compute(const TileSrc& src, const PairRec& 
   const double2 g0 = (k.geo + t.ket0)[lane_off], g1 = (k.geo + k.npairs + t.ket0)[lane_off];
   const double ACx = bp.A[0] - g0.x, ACy = bp.A[1] - g0.y, ACz = bp.A[2] - g1.x;
   const PairRec& k0 = src.pairs[t.ket0];
-  const int knp = k0.np, kps = k0.ps, row = k0.p0;
+  const int kps = k0.ps, row = k0.p0;
   const PrimRec* __restrict__ bprim = prim + bp.p0;
-  const int bnp = bp.np, bps = bp.ps;
-  for (int j = 0; j < knp; ++j) {
+  const int bps = bp.ps;
+  int i0 = 0, i1 = bp.np, j0 = 0, j1 = k0.np;
+  if (t.pad != 0) {  // a part of the quartets' primitives (PrimSplit)
+    i0 = t.pad & 255;
+    i1 = (t.pad >> 8) & 255;
+    j0 = (t.pad >> 16) & 255;
+    j1 = (t.pad >> 24) & 255;
+  }
+  for (int j = j0; j < j1; ++j) {
     const PrimRec pk = load_ket_prim<double, true>(k, prim, row + j * kps, lane_off);
     const double QAx = pk.pax - ACx, QAy = pk.pay - ACy, QAz = pk.paz - ACz;
-    for (int i = 0; i < bnp; ++i) {
+    for (int i = i0; i < i1; ++i) {
       const PrimRec pb = bprim[i * bps];
       const double rs = fast_rsqrt(pb.zeta + pk.zeta);  // (zeta + eta)^(-1/2)
       const double ooze = rs * rs;
@@ -169,7 +180,6 @@ __global__ __launch_bounds__(THREADS, MINW) void eri_part_kernel(
     }
     for (int ti = ch.tb; ti < ch.te; ++ti) {
       const Tile t = tiles[ti];
-      if (!first_part(t.pad)) continue;  // the first part does the whole quartets
       const bool active = lane < t.count;
       const int lane_off = active ? lane : 0;  // an idle lane repeats the first
       part_run<LA, LB, LC, LD, 0>(wave, src, bp, t, lane, lane_off, part_lds, prims, slab);

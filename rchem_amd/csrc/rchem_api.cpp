@@ -1345,6 +1345,17 @@ int split_limit(const QClass& qc, double iters) {
   const int floor = 16 >> std::min(2, qc.la + qc.lb + qc.lc + qc.ld);
   return std::max(floor, static_cast<int>(std::min(1e9, iters / 2048.0)));
 }
+// The same for the partwise kernels, whose tile is a workgroup's: twice a compute
+// unit's share of the class, and not below 8 (a part costs its horizontal
+// recurrences and digestion, some 2 primitive quartets).  Builds in ms with tiles
+// whole, by these, with half and twice the share, with a floor of 16:
+// 5 d and 5 p shells of 6 primitives 66.1, 6.9, 7.6, 12.8, 6.9; one of each 19.8,
+// 0.77, 0.78, 0.80, 0.76; 12 s/p/d shells of 3 primitives 4.36, 1.08, 1.09, 1.11,
+// 1.19, 48 of them 6.56, 3.05, 3.49, 3.24, 3.06, 96 12.6, 11.2, 11.1, 11.2, 11.2.
+// (The engines before them, a wave to a quartet, took 26.4, 6.5, 3.15, 13.9, 26.)
+int part_split_limit(double iters, int cus) {
+  return static_cast<int>(std::max(8.0, std::min(1e9, 2.0 * iters / cus)));
+}
 // A workgroup takes a chunk's tiles in turn, so a class's chunks are at most its
 // tiles / 1024 (at least 8): (H2O)_8 1.06 -> 0.84 ms, water 0.26 -> 0.19.
 constexpr double kMinChunks = 1024.0;
@@ -1421,8 +1432,12 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
     if (qc.quartets > 0)
       TRY(class_kernel(ctx, qc.la, qc.lb, qc.lc, qc.ld, kModeJK, kBoysExact, 0, &k));
     partwise[c] = k.part;
-    if (!k.fn) continue;  // the other engines spread a quartet over a wave
-    limit[c] = split_limit(qc, iters[c]);
+    if (k.part.launch)
+      limit[c] = part_split_limit(iters[c], ctx->cus);
+    else if (k.fn)
+      limit[c] = split_limit(qc, iters[c]);
+    else
+      continue;  // the other engines spread a quartet over a wave
     if (limit[c] >= npmax[c]) limit[c] = 0;
     if (limit[c] > 0) {
       split = true;
@@ -1460,8 +1475,12 @@ int prepare_plan(rchem_ctx* ctx, double tau) {
   for (size_t c = 0; c < nq; ++c) {
     double tiles = 0.0;
     for (const double x : bra_cap[c]) tiles += x;
-    if (partwise[c].launch) {  // a chunk to a workgroup, one workgroup a CU
-      chunk_most[c] = static_cast<int>(std::min(4096.0, std::max(4.0, tiles / (16.0 * ctx->cus))));
+    if (partwise[c].launch) {  // a chunk to a workgroup
+      // a few chunks to a workgroup, and of four tiles (a chunk's K rows are
+      // cleared and flushed) once each has some
+      const double cu = tiles / ctx->cus;
+      chunk_most[c] = static_cast<int>(
+          std::min(4096.0, std::max(std::clamp(cu / 2.0, 1.0, 4.0), cu / 16.0)));
       slab = std::max(slab, partwise[c].slab * static_cast<size_t>(std::max(
                                 1.0, std::min(tiles, 1.0 * ctx->cus * partwise[c].groups))));
       continue;
