@@ -1,15 +1,14 @@
 // Device Boys function F_m(T) = int_0^1 t^(2m) exp(-T t^2) dt for gfx950.
 //
 // Two evaluations:
-//   * exact (production): F_M(T) from a polynomial about the centre of T's grid
-//     cell, then downward recursion F_m = (2T F_{m+1} + e^{-T}) / (2m+1), which
-//     is stable, with e^{-T} = e^{-T0} e^{T0 - T} from the same cell and a short
+//   * exact (production): F_M(T) from a polynomial about the grid point nearest to
+//     T, then downward recursion F_m = (2T F_{m+1} + e^{-T}) / (2m+1), which
+//     is stable, with e^{-T} = e^{-T0} e^{T0 - T} from the same row and a short
 //     polynomial.  For T >= 36 the asymptote F_0 = sqrt(pi/T)/2 (error < e^{-T})
 //     and the upward recursion F_{m+1} = ((2m+1) F_m - e^{-T}) / (2T) are used.
-//     The coefficients are the Taylor series about the cell's centre with its
-//     last terms folded down (Chebyshev economisation), computed on the host in
-//     long double; a kernel stages its order's block in LDS, so every lookup is
-//     an LDS read, not a cache miss.
+//     The coefficients are computed on the host in long double (boys_table.hpp); a
+//     kernel stages its order's block in LDS, so every lookup is an LDS read, not
+//     a cache miss.
 //   * compat (parity with the reference): the Numerical-Recipes incomplete
 //     gamma of libpyquante2 (cints.c:302-373) evaluated per m with its own
 //     constants (EPS = 3e-7, ITMAX = 100, x clamped to >= 1e-8), so integrals
@@ -18,67 +17,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "boys_layout.hpp"
+
 namespace rchem {
-
-constexpr int kBoysMaxM = 9;                          // highest m served
-constexpr double kBoysTMax = 36.0;
-
-// The grid.  A lookup gathers one row of coefficients per lane, and those
-// gathers (random rows, so each LDS instruction meets bank conflicts) kept the
-// LDS busy for 44 % of the (10|00) and (00|00) kernels' time when a row was 9
-// Taylor coefficients on a uniform grid of 1/8.  Cutting the series of a cell
-// of half width h at n terms leaves h^n F_{m+n} / n! 2^(1-n) of it in Chebyshev
-// polynomials, 2^(1-n) of what cutting the powers of d leaves.
-//   * orders 0 and 1: F_{m+n} / F_m falls as T^-n beyond T ~ 4, so cells that
-//     double in width from one octave of T + 4 to the next ([4, 8), [8, 16),
-//     [16, 32), [32, 40)) need the same n everywhere: 13/4 octaves of 2^bits
-//     cells where a uniform grid has 36/4.  FP64: 2^6 cells to an octave (width
-//     1/16 below T = 4; 208 rows, 12 and 15 KB of LDS where 289 rows took 21)
-//     and 7 terms for order 0, 8 for order 1.  FP32: 4 terms, one 16-byte read.
-//   * orders >= 2: the fall begins later (T > m + n), so the grid stays uniform:
-//     FP64 1/8 with 8 terms, FP32 1/16 with 4.
-// Worst relative errors over 0 <= T < 36 against 80-bit F_m (3e5 arguments, log
-// and uniform, cell edges among them; the 9-term rows in brackets): order 0
-// 2.5e-16 (2.1e-16; 2.1e-16 outside the two cells above T = 12), order 1 F_0
-// 2.1e-16 (2.1e-16) and F_1 7.0e-16 (1.1e-15), order 4 F_0 6.8e-16 (6.8e-16)
-// and F_4 2.2e-16 (2.2e-16).  FP32: order 0 1.1e-7 (1.1e-7), F_1 1.6e-7
-// (1.6e-7), order 4 F_0 4.3e-7 (4.3e-7).
-__host__ __device__ constexpr bool boys_octaves(int M) { return M <= 1; }
-__host__ __device__ constexpr int boys_bits(int M, bool f64) { return f64 || M == 0 ? 6 : 8; }
-__host__ __device__ constexpr int boys_inv_h(bool f64) { return f64 ? 8 : 16; }
-__host__ __device__ constexpr int boys_terms(int M, bool f64) {
-  return f64 ? (M == 0 ? 7 : 8) : 4;
-}
-// Entries from one row to the next: FP64 rows an odd number of doubles (8-term
-// rows padded to 9), so that rows start at every bank pair.
-__host__ __device__ constexpr int boys_stride(int M, bool f64) {
-  return f64 ? (M == 0 ? 7 : 9) : 4;
-}
-__host__ __device__ constexpr int boys_rows(int M, bool f64) {
-  return boys_octaves(M) ? 13 << (boys_bits(M, f64) - 2)  // three octaves and [32, 40)
-                         : 36 * boys_inv_h(f64) + 1;
-}
-__host__ __device__ constexpr int boys_block(int M, bool f64) {
-  return boys_rows(M, f64) * boys_stride(M, f64);
-}
-// Device layout: the orders' blocks one after the other, then (FP64) the row
-// of e^{-T0} that the downward recursions of M >= 2 share.  Order 1 holds F_0
-// as a polynomial whose derivative is F_1 (dF_0/dT = -F_1), so that one pass
-// gives both with no exponential.
-__host__ __device__ constexpr int boys_offset(int M, bool f64) {
-  int o = 0;
-  for (int m = 0; m < M; ++m) o += boys_block(m, f64);
-  return o;
-}
-constexpr int kBoysExpRows = boys_rows(2, true);
-constexpr int kBoysExpOffset = boys_offset(kBoysMaxM + 1, true);
-constexpr int kBoysTableSize = kBoysExpOffset + kBoysExpRows;
-constexpr int kBoysTableSizeF = boys_offset(kBoysMaxM + 1, false);
-// Staged entries a kernel of highest order M needs: its block and, for FP64
-// and M >= 2, the exp row.
-__host__ __device__ constexpr int boys_stage_size(int M, bool f64 = true) {
-  return boys_block(M, f64) + (f64 && M >= 2 ? kBoysExpRows : 0);
-}
 
 enum BoysMode { kBoysExact = 0, kBoysCompat = 1 };
 
@@ -98,81 +39,56 @@ __device__ __forceinline__ double fast_rsqrt(double x) {
 }
 __device__ __forceinline__ float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 
-// The cell of T (0 <= T < kBoysTMax) on the grid of 2^BITS cells to an octave
-// of T + 4, and d = T0 - T, T0 the cell's centre.  The sum r = T + 4 has the
-// octave in its exponent and the cell in its leading BITS mantissa bits: the
-// row index is its high word shifted, the centre that word with the rest
-// replaced by 100...0.  T0 - T is exact, so rounding r costs nothing but a cell
-// entered an ulp early.  r < 40 for every T < 36 (ulps are equal there).
-template <int BITS, typename R>
-__host__ __device__ __forceinline__ void boys_cell(R T, int* k, R* d) {
-  const R r = T + R(4);
-  if constexpr (sizeof(R) == 8) {
-    constexpr int sh = 20 - BITS;
-    union { double f; unsigned long long u; } x{r}, c;
-    const unsigned hi = static_cast<unsigned>(x.u >> 32);
-    *k = static_cast<int>(hi >> sh) - (0x40100000 >> sh);
-    c.u = static_cast<unsigned long long>((hi & (~0u << sh)) | (1u << (sh - 1))) << 32;
-    *d = (c.f - 4.0) - T;
-  } else {
-    constexpr int sh = 23 - BITS;
-    union { float f; unsigned u; } x{r}, c;
-    *k = static_cast<int>(x.u >> sh) - (0x40800000 >> sh);
-    c.u = (x.u & (~0u << sh)) | (1u << (sh - 1));
-    *d = (c.f - 4.0f) - T;
-  }
-}
-
-// The grid point nearest to T (0 <= T < kBoysTMax) of the uniform grid: its
-// index k and d = T0 - T, |d| at most half the spacing.  Rounding by adding the
-// power of two whose ulp is the spacing: the sum r = kMagic + T0 has k in its
-// low mantissa bits (read off the register, no conversion), r - kMagic is T0
-// exactly, and T0 - T is exact (a multiple of T's ulp).  A tie rounds to even.
-template <typename R>
-__host__ __device__ __forceinline__ void boys_grid(R T, int* k, R* d) {
+// The grid point nearest to T (0 <= T < kBoysTMax): its index k and d = T0 - T,
+// |d| at most half the spacing.  Rounding by adding the power of two whose ulp is
+// the spacing: the sum r = kMagic + T0 has k in its low mantissa bits (read off the
+// register, no conversion), r - kMagic is T0 exactly, and T0 - T is exact (a
+// multiple of T's ulp).  A tie rounds to even.
+template <int M, typename R>
+__host__ __device__ __forceinline__ void boys_locate(R T, int* k, R* d) {
+  constexpr int inv_h = boys_inv_h(M, sizeof(R) == 8);
   if constexpr (sizeof(R) == 8) {
     constexpr double kMagic = 562949953421312.0;  // 2^49: ulp 1/8 on [2^49, 2^50)
-    static_assert(boys_inv_h(true) == 8, "kMagic");
+    static_assert(inv_h == 8, "kMagic");
     const union { double f; unsigned long long u; } r{T + kMagic};
     *k = static_cast<int>(static_cast<unsigned>(r.u));
     *d = (r.f - kMagic) - T;
   } else {
-    constexpr float kMagic = 524288.0f;  // 2^19: ulp 1/16 on [2^19, 2^20)
-    static_assert(boys_inv_h(false) == 16, "kMagic");
+    // 2^20 and 2^19: ulps 1/8 and 1/16 up to the next power
+    constexpr float kMagic = inv_h == 8 ? 1048576.0f : 524288.0f;
+    static_assert(inv_h == 8 || inv_h == 16, "kMagic");
     const union { float f; unsigned u; } r{T + kMagic};
     *k = static_cast<int>(r.u & 0x7fffffu);
     *d = (r.f - kMagic) - T;
   }
 }
 
-// Row and offset of T in the block of order M.
-template <int M, typename R>
-__host__ __device__ __forceinline__ void boys_locate(R T, int* k, R* d) {
-  if constexpr (boys_octaves(M)) boys_cell<boys_bits(M, sizeof(R) == 8), R>(T, k, d);
-  else boys_grid<R>(T, k, d);
-}
-
-// e^d, |d| <= 1/16, by its Taylor series (the recursion multiplies its error,
-// so it keeps the ninth term that F_M's polynomial does without).
+// e^d, |d| <= 1/16, by its Taylor series.
 constexpr int kExpTerms = 9;
 constexpr double kExpPoly[kExpTerms] = {1.0,       1.0,       1.0 / 2,    1.0 / 6,    1.0 / 24,
                                         1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320};
 
-// The coefficients of row k of a staged block of order M (FP32 rows are 16-byte
-// aligned: one wide LDS read).
+// The coefficients of row k of a staged block of order M (FP32 rows are read in
+// their 16 bytes or, of 24, in eights).
 template <int M, typename R>
 __device__ __forceinline__ void boys_row(const R* __restrict__ table, int k, R* __restrict__ c) {
   constexpr int K = boys_terms(M, sizeof(R) == 8);
   // 0 <= k < rows: a 24-bit multiply (full rate; a 32-bit one is quarter rate)
-  const R* __restrict__ row =
-      table + __umul24(static_cast<unsigned>(k), boys_stride(M, sizeof(R) == 8));
-  if constexpr (sizeof(R) == 4) {
-    static_assert(K == 4 || sizeof(R) == 8, "one float4 per FP32 row");
+  const R* __restrict__ row = table + __umul24(static_cast<unsigned>(k), K);
+  if constexpr (sizeof(R) == 4 && K == 4) {
     const float4 v = *reinterpret_cast<const float4*>(row);
     c[0] = v.x;
     c[1] = v.y;
     c[2] = v.z;
     c[3] = v.w;
+  } else if constexpr (sizeof(R) == 4) {
+    static_assert(sizeof(R) == 8 || K % 2 == 0, "rows of whole float2");
+#pragma unroll
+    for (int j = 0; j < K; j += 2) {
+      const float2 v = *reinterpret_cast<const float2*>(row + j);
+      c[j] = v.x;
+      c[j + 1] = v.y;
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < K; ++j) c[j] = row[j];

@@ -50,36 +50,29 @@ __host__ __device__ __forceinline__ int rec_fields(int L) { return kG + L + 1; }
 
 // pref * F_m(T), m = 0..M, into out[m * stride]: the exact Boys function with
 // the order a run-time value, from the device table (boys.hpp: the row of T's
-// cell, the exp row, downward recursion; asymptote and upward recursion for
+// grid point, the exp row, downward recursion; asymptote and upward recursion for
 // T >= 36).
 __device__ void boys_exact_strided(int M, double T, const double* __restrict__ table, double pref,
                                    double* __restrict__ out, int stride) {
   if (T < kBoysTMax) {
+    constexpr int K = boys_terms(0, true);
     int k;
     double d;
-    if (M == 0) {
-      boys_locate<0, double>(T, &k, &d);
-      const double* c = table + k * boys_stride(0, true);
-      double f = c[boys_terms(0, true) - 1];
-      for (int j = boys_terms(0, true) - 2; j >= 0; --j) f = c[j] + d * f;
-      out[0] = pref * f;
-      return;
-    }
+    boys_locate<0, double>(T, &k, &d);  // every order's grid
+    const double* c = table + M * boys_block(0, true) + k * K;
     if (M == 1) {
-      boys_locate<1, double>(T, &k, &d);
       double f0, f1;
-      boys_poly01<boys_terms(1, true)>(table + boys_offset(1, true) + k * boys_stride(1, true), d,
-                                       &f0, &f1);
+      boys_poly01<K>(c, d, &f0, &f1);
       out[0] = pref * f0;
       out[stride] = pref * f1;
       return;
     }
-    constexpr int K = boys_terms(2, true);
-    boys_locate<2, double>(T, &k, &d);
-    const double* c =
-        table + boys_offset(2, true) + (M - 2) * boys_block(2, true) + k * boys_stride(2, true);
     double f = c[K - 1];
     for (int j = K - 2; j >= 0; --j) f = c[j] + d * f;
+    if (M == 0) {
+      out[0] = pref * f;
+      return;
+    }
     double pe = kExpPoly[kExpTerms - 1];
     for (int j = kExpTerms - 2; j >= 0; --j) pe = kExpPoly[j] + d * pe;
     const double e = table[kBoysExpOffset + k] * pe;

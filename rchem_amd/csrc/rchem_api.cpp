@@ -23,6 +23,7 @@
 
 #include "../../include/rchem_gpu.h"
 #include "boys.hpp"
+#include "boys_table.hpp"
 #include "tile_width.hpp"
 #include "types.hpp"
 
@@ -493,104 +494,8 @@ void set_global_error(const std::string& msg) { g_create_error = msg; }
 
 namespace {
 
-// The Boys tables in device layout (boys.hpp).  Per cell: the derivatives of
-// F_M about the centre T0, F_{M+j}(T0) / j! in powers of T0 - T, from the
-// all-positive series F_m(T) = e^{-T} sum_k (2T)^k / ((2m+1) ... (2m+2k+1)) at
-// the highest order and downward recursion, in long double; the series is
-// rewritten in Chebyshev polynomials of the cell and cut there, which leaves
-// 2^(1-n) of what cutting the powers would.  Order 1 cuts the series of F_1 and
-// integrates it, so that F_0's polynomial starts at F_0(T0) exactly and has
-// F_1's as its derivative.
-struct BoysTables {
-  std::vector<double> f64;
-  std::vector<float> f32;
-};
-
 const BoysTables& boys_tables() {
-  static const BoysTables tables = [] {
-    constexpr int kD = 14;  // terms of the series before the cut
-    constexpr int kM = kBoysMaxM + kD;
-    using Real = long double;
-    // Chebyshev polynomials' coefficients
-    static Real cheb[kD][kD] = {};
-    cheb[0][0] = 1.0L;
-    cheb[1][1] = 1.0L;
-    for (int n = 2; n < kD; ++n)
-      for (int i = 0; i < kD; ++i)
-        cheb[n][i] = (i > 0 ? 2.0L * cheb[n - 1][i - 1] : 0.0L) - cheb[n - 2][i];
-    auto boys_at = [](Real T, Real* F) {
-      Real term = 1.0L / (2 * kM + 1), sum = term;
-      for (int k = 1; k < 4000; ++k) {
-        term *= 2.0L * T / (2 * kM + 2 * k + 1);
-        sum += term;
-        if (term < sum * 1e-21L) break;
-      }
-      const Real e = expl(-T);
-      F[kM] = e * sum;
-      for (int m = kM - 1; m >= 0; --m) F[m] = (2.0L * T * F[m + 1] + e) / (2 * m + 1);
-    };
-    // the first K coefficients in d of sum_j a_j d^j over |d| <= h, cut in
-    // Chebyshev polynomials of d / h
-    auto cut = [](const Real* a, Real h, int K, Real* out) {
-      Real r[kD], keep[kD] = {};
-      Real hp = 1.0L;
-      for (int j = 0; j < kD; ++j, hp *= h) r[j] = a[j] * hp;
-      for (int n = kD - 1; n >= 0; --n) {
-        const Real c = r[n] / cheb[n][n];
-        for (int i = 0; i <= n; ++i) {
-          r[i] -= c * cheb[n][i];
-          if (n < K) keep[i] += c * cheb[n][i];
-        }
-      }
-      hp = 1.0L;
-      for (int j = 0; j < K; ++j, hp *= h) out[j] = keep[j] / hp;
-    };
-    BoysTables t;
-    t.f64.resize(kBoysTableSize);
-    t.f32.resize(kBoysTableSizeF);
-    for (const bool f64 : {true, false})
-      for (const int first : {0, 1, 2}) {  // orders with a grid of their own: 0, 1, 2 and above
-        const int last = first < 2 ? first : kBoysMaxM, bits = boys_bits(first, f64);
-        for (int r = 0; r < boys_rows(first, f64); ++r) {
-          Real h, T;  // half width and centre of cell r
-          if (boys_octaves(first)) {
-            const Real octave = ldexpl(4.0L, r >> bits);
-            h = ldexpl(octave, -bits - 1);
-            T = octave + (2 * (r & ((1 << bits) - 1)) + 1) * h - 4.0L;
-          } else {
-            h = 0.5L / boys_inv_h(f64);
-            T = static_cast<Real>(r) / boys_inv_h(f64);
-          }
-          Real F[kM + 1];
-          boys_at(T, F);
-          for (int M = first; M <= last; ++M) {
-            const int K = boys_terms(M, f64);
-            Real a[kD], c[kD], fact = 1.0L;
-            for (int j = 0; j < kD; ++j) {
-              if (j > 0) fact *= j;
-              a[j] = F[M + j] / fact;
-            }
-            if (M == 1) {
-              Real q[kD];
-              cut(a, h, K - 1, q);
-              c[0] = F[0];
-              for (int j = 1; j < K; ++j) c[j] = q[j - 1] / j;
-            } else {
-              cut(a, h, K, c);
-            }
-            const size_t o = boys_offset(M, f64) + static_cast<size_t>(r) * boys_stride(M, f64);
-            for (int j = 0; j < K; ++j) {
-              if (f64)
-                t.f64[o + j] = static_cast<double>(c[j]);
-              else
-                t.f32[o + j] = static_cast<float>(c[j]);
-            }
-          }
-          if (f64 && first == 2) t.f64[kBoysExpOffset + r] = static_cast<double>(expl(-T));
-        }
-      }
-    return t;
-  }();
+  static const BoysTables tables = make_boys_tables();
   return tables;
 }
 
