@@ -2786,9 +2786,12 @@ int scf_run(rchem_ctx* ctx, int natom, const double* Z, const double* xyz,
   HIPC(dflag.ensure(sizeof(double) * 2 * kSmallSteps));
   if (small) HIPC(fill_launch(dflag.as<double>(), 2 * kSmallSteps, 1.0, ctx->stream));
   DevBuf dP, dP2, dP3, dpl, dph, dpar, dsp2;
-  // above that, up to kSp2MaxN (where the library's products on the whole chip
-  // become the better ones), a step is one launch
-  constexpr int kSp2MaxN = 1024;
+  // above that, up to kSp2MaxN, a step is one launch; beyond, the library's
+  // products on the whole chip are the better ones.  14 iterations of a mixed SCF
+  // (graph / kernel by kernel) by steps and by products, ms: n = 624 222 / 208 and
+  // 228 / 229, 728 289 / 278 and 288 / 282, 832 381 / 351 either way, 1014
+  // 573 / 557 and 546 / 530
+  constexpr int kSp2MaxN = 832;
   const bool sp2 = opts->purify && !small && n <= kSp2MaxN && opts->nocc < n;
   if (opts->purify && !small) {
     HIPC(dP.ensure(n2 * sizeof(double)));
