@@ -551,9 +551,11 @@ __global__ __launch_bounds__(256) void eri_kernel(
     const float4* __restrict__ kprim4, const float2* __restrict__ kprim2) {
   // Other modes than kModeJK read their records through the argument struct:
   // with the restrict-qualified arrays the compat kernels of (dp|ds) and
-  // (dd|ds), whose 512 registers spill, returned a few wrong integrals
-  // (deterministic, the same instruction stream otherwise correct: a compiler
-  // fault), and no caller of theirs is bound by these loads.
+  // (dd|ds), whose 512 registers spill, returned a few wrong integrals, the same
+  // ones every time.  The cause was not found.  No caller of these modes is bound
+  // by the loads.  (The Fock-build kernels of the same classes, which do read the
+  // qualified arrays, are held to the tensor's integrals and to the oracle's by the
+  // d-class and partwise tests.)
   const TileSrc src{MODE == kModeJK ? pairs : a.pairs, MODE == kModeJK ? tiles : a.tiles,
                     KetPlanes{kgeo, kfn, kprim, kprim4, kprim2, a.ket.npairs, a.ket.nprims}};
   const typename PrimOf<R>::T* __restrict__ prim = prims_of<R>(prims, prims_f);

@@ -373,8 +373,8 @@ struct rchem_ctx {
   double pairs_tau = -1.0;
   std::vector<PairRec> pairs;
   std::vector<double> pairQ;                      // Schwarz bound, layout order
-  std::vector<std::pair<int, int>> pair_shells;
-  std::vector<double> pair_kmax;  // max |K_ab| of each pair's primitive pairs (layout order)   // (a, b), layout order
+  std::vector<std::pair<int, int>> pair_shells;   // (a, b), layout order
+  std::vector<double> pair_kmax;                  // max |K_ab| of each pair's primitive pairs, layout order
   size_t nprims = 0;
   std::vector<Bucket> buckets[kNumPairClasses];
   int class_begin[kNumPairClasses + 1] = {0};
@@ -1824,13 +1824,13 @@ int jk_device(rchem_ctx* ctx, const double* dD, double* dJ, double* dK, const rc
       a.jp_bra = ctx->jp_cls[qc.X];
       a.jp_ket = ctx->jp_cls[qc.Y];
       a.Dp = bf.dp;
-      // K rows of the bra pair in LDS when they fit in 64 KB: every column, or
-      // the bra's molecule's window in a multi-molecule basis
+      // K rows of the bra pair: every column, or the bra's molecule's window in a
+      // multi-molecule basis
       const bool multi = !ctx->shell_mol.empty();
       a.kw = multi ? ctx->mol_kw : ctx->nbf;
       a.pair_kc0 = multi ? ctx->pair_kc0_d.as<int>() : nullptr;
       // K rows in LDS when they fit the device's LDS per workgroup beside the
-      // kernel's own arrays (Boys block, bra primitive pairs: < 12 KB)
+      // kernel's own arrays
       const size_t lds = sizeof(double) * (ncart(qc.la) + ncart(qc.lb)) * static_cast<size_t>(a.kw);
       const bool lds_ok = lds + kLdsStaticReserve <= ctx->lds_block && ctx->lds_digestion &&
                           !ctx->force_generic &&

@@ -245,14 +245,14 @@ hipError_t antisym_launch(const double* A, double* E, int n, hipStream_t s) {
 }  // namespace rchem
 
 namespace rchem {
-// Start of the purification of F (n x n, symmetric) for nocc occupied
-// orbitals: P = P_0.  lo, hi: n doubles of scratch; par: 3 doubles.
 // Gershgorin's bounds of every row of F.
 hipError_t gersh_launch(const double* F, int n, double* lo, double* hi, hipStream_t s) {
   hipLaunchKernelGGL(gersh_kernel, dim3((n + 3) / 4), dim3(256), 0, s, F, n, lo, hi);
   return hipGetLastError();
 }
 
+// Start of the purification of F (n x n, symmetric) for nocc occupied
+// orbitals: P = P_0.  lo, hi: n doubles of scratch; par: 3 doubles.
 hipError_t purify_start_launch(const double* F, int n, int nocc, double* lo, double* hi,
                                double* par, double* P, hipStream_t s) {
   hipLaunchKernelGGL(gersh_kernel, dim3((n + 3) / 4), dim3(256), 0, s, F, n, lo, hi);
