@@ -13,7 +13,8 @@
 // digests them before the next ab, so that one ab's integrals are live at a time.
 // K goes to rows of a and b in LDS, the ket's Coulomb sums of all waves to LDS
 // too: with every sum an atomic in memory the kernels ran at 40 to 60e9 atomics/s
-// whatever their arithmetic ((dp|pp) 47.5 ms against 19.2, (dd|dp) 29 against 18.5).
+// whatever their arithmetic ((dp|pp), in eight parts then, 47.5 ms against 19.2,
+// (dd|dp) 29 against 18.5).
 //
 // The per-lane kernels spilled (512 registers and up to 1.2 KB a lane), and the
 // streaming kernel (eri_stream.hpp: one wave to a quartet, lanes on its
@@ -24,9 +25,9 @@
 // with the product and Boys work that each part repeats (130 of 535 vector
 // instructions of a (dp|dp) part) the larger part of the excess.  A build of 210
 // s/p/d shells of 3 primitives (n = 430), ms, per-lane or streaming and now:
-// (dp|pp) 17.6, 15.5; (dp|dp) 68.6, 16.2; (dd|ds) 20.5, 8.9; (dd|pp) 42.0, 8.6;
-// (dd|dp) 55.0, 18.1; (dd|dd) 32.0, 6.9.  The build: 271 -> 133, and 127 with the
-// chunks handed out by a counter.
+// (dp|pp) 17.6, 13.5; (dp|dp) 68.6, 14.2; (dd|ds) 20.5, 7.0; (dd|pp) 42.0, 7.6;
+// (dd|dp) 55.0, 14.6; (dd|dd) 32.0, 6.5.  The build: 298 -> 132 on one box (108 to
+// 132 over boxes).
 //
 // A tile is one lane's chain of primitive quartets, so where a class has fewer
 // tiles than the chip workgroups they are split over the primitives as in the

@@ -9,8 +9,14 @@
 // with Gershgorin's bounds, then P <- P^2 or 2P - P^2, whichever brings the trace
 // nearer to nocc (the trace-correcting second-order scheme, Niklasson 2002;
 // every step squares the distance of the eigenvalues from 0 or from 1).  A
-// matrix without a gap at the Fermi level does not get there; its flag stays 0
+// matrix without a gap at the Fermi level does not get there; its flag says so
 // and the caller takes the eigensolver.
+//
+// Error against extended precision of the density of a core guess, 56 matrices of 1
+// to 8 waters (n = 7 to 104, gaps 0.2 to 4): the largest 1.07 times rocSOLVER's
+// eigensolver's in the geometric mean (0.63 to 2.0; 2.5e-15 to 3e-13, most of it
+// S^(-1/2)'s), the root mean square 1.00 times; the cubic scheme by library products
+// 1.07 times.  (Dense synthetic spectra with core levels at -20: up to 7 times.)
 //
 // What bounds it: one matrix's products on one CU.  The matrix stays in LDS
 // (128 x 130 doubles) from F' to P; a step is the lower triangle of P^2 on the
